@@ -451,547 +451,4 @@ __global__ __launch_bounds__(256) void k_reduce_parts(const ReduceItem* __restri
   }
 }
 
-// ------------------------------------------------------------------------------------------
-// The diagonal block of a panel: factored column by column with the reference's pivot test
-// (cholesky.rs:1146-1171: a pivot not above 1e-10 |A_jj|, or not finite, fails the column),
-// then inverted, Linv = L11^-1, for the rows below (a GEMM). The arithmetic is FP64 whatever
-// the storage. Item: f, a = c0; Linv goes to the panel's slot in Inv (F.inv0 + (c0 / NB) NB^2).
-
-constexpr double PIVOT_TOL = 1e-10;  // cholesky.rs:48
-
-// ------------------------------------------------------------------------------------------
-// The diagonal block of a panel (any width up to NB): it splits into halves of h0 = 64 and
-// h1 = pw - 64 columns (h1 = 0 for panels up to 64 wide),
-//   [A11    ]   [L11    ] [L11^T L21^T]          [X11    ]
-//   [A21 A22] = [L21 L22] [      L22^T],  Linv = [X21 X22],  X21 = -X22 L21 X11,
-// Each half is factored and inverted inside one wave (wave_potrf_inv): the column values pass
-// between lanes by shuffles, so the 128 sequential column steps need no workgroup barrier and
-// wait on no memory. Everything else is a 64 x 64 x 64 product on the FP64 MFMA with its
-// operands read from LDS (strip64, a 64 x 16 strip per wave):
-// L21 = A21 X11^T, A22 -= L21 L21^T, T = L21 X11, X21 = -X22 T.
-//
-// LDS holds the block in FP64: S[i][j] = L(i, j) for i >= j and Linv(j, i) for i < j, the
-// inverse's diagonal in xd. The pivot test is the reference's. Outputs: L11 over the block's lower
-// triangle in L, and Linv (pw x pw, column-major, zeros above the diagonal) in its slot of Inv.
-
-// Wave-local Cholesky and inverse of the h x h block at S[o.., o..] (h <= 64), the wave as an
-// 8 x 8 lane grid: lane (ti, tk) = (lane % 8, lane / 8) holds a[r][c] = A(ti + 8 r, tk + 8 c)
-// and x[r][c] = X(ti + 8 r, tk + 8 c). Step j scales column j of L and broadcasts it by
-// shuffles (the trailing update is then local), and takes the same step of the inverse,
-// right-looking on L X = I: row j of X is divided by L(j, j), then X(i, :) -= L(i, j) X(j, :)
-// for i > j. Lane 0 applies the pivot test and records the first failing column.
-// Steps 8 CB .. 8 CB + 7 (a template, so that every register index is a constant). Only the
-// 8 x 8 register blocks the step can change are touched: (r, c) with r >= c >= CB for L and
-// r >= CB, c <= CB for X; within them the remaining conditions are per-lane selects, not
-// branches.
-// A double from one lane (uniform index) to the whole wave, by scalar reads of its halves.
-__device__ __forceinline__ double readlane_d(double v, int l) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, l);
-  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// EXACT (FP64 storage): d = sqrt(p) and column / d, correctly rounded like the reference.
-// Otherwise (FP32 storage) the step takes rd from the hardware reciprocal square root with two
-// Newton steps and multiplies: the values are rounded to FP32 afterwards, and the step's
-// dependent chain (the part that sets this kernel's time) is shorter.
-template <int CB, bool EXACT, int NBK>
-__device__ __forceinline__ void wpi_steps(double (&a)[NBK][NBK], double (&x)[NBK][NBK], int h, int lane, double dl,
-                                          int64_t col, unsigned long long* __restrict__ fail, bool& bad) {
-  const int ti = lane & 7, tk = lane >> 3;
-  for (int cc = 0; cc < 8; ++cc) {
-    const int j = 8 * CB + cc;
-    if (j >= h) return;
-    const double p = readlane_d(a[CB][CB], cc + 8 * cc);  // the pivot, on the step's dependent chain
-    const double a0 = readlane_d(dl, j);
-    if (lane == 0 && !bad && (!(p > PIVOT_TOL * a0) || !isfinite(p))) {
-      atomicMin(fail, (unsigned long long)(col + j));
-      bad = true;
-    }
-    double d, rd;
-    if constexpr (EXACT) {
-      d = sqrt(p);
-      rd = 1.0 / d;
-    } else {
-      const double y = __builtin_amdgcn_rsq(p), hp = 0.5 * p;
-      const double y1 = y * fma(-hp * y, y, 1.5);
-      rd = y1 * fma(-hp * y1, y1, 1.5);
-      d = p * rd;
-    }
-    {  // column j of L: rows below scaled, the pivot replaced by d (lanes tk == cc own it)
-      const bool own = tk == cc;
-#pragma unroll
-      for (int r = CB; r < NBK; ++r) {
-        const bool below = r > CB || ti > cc, diag = r == CB && ti == cc;
-        const double sc = EXACT ? a[r][CB] / d : a[r][CB] * rd;
-        a[r][CB] = own ? (below ? sc : (diag ? d : a[r][CB])) : a[r][CB];
-      }
-    }
-    {  // row j of X divided by L(j, j) (lanes ti == cc own it)
-      const bool own = ti == cc;
-#pragma unroll
-      for (int c = 0; c <= CB; ++c) x[CB][c] = own ? x[CB][c] * rd : x[CB][c];
-    }
-    double li[NBK], lk[NBK], xj[NBK];
-#pragma unroll
-    for (int r = CB; r < NBK; ++r) li[r] = __shfl(a[r][CB], ti + 8 * cc);  // L(ti + 8r, j)
-#pragma unroll
-    for (int c = CB; c < NBK; ++c) lk[c] = __shfl(a[c][CB], tk + 8 * cc);  // L(tk + 8c, j)
-#pragma unroll
-    for (int c = 0; c <= CB; ++c) xj[c] = __shfl(x[CB][c], cc + 8 * tk);  // X(j, tk + 8c)
-    const bool kj = tk > cc, ik = ti >= tk, ij = ti > cc;
-#pragma unroll
-    for (int r = CB; r < NBK; ++r) {
-#pragma unroll
-      for (int c = CB; c <= r; ++c) {  // L(i, k) -= L(i, j) L(k, j) for i >= k > j
-        const bool upd = (c > CB || kj) && (r > c || ik);
-        const double t = fma(-li[r], lk[c], a[r][c]);
-        a[r][c] = upd ? t : a[r][c];
-      }
-      const bool below = r > CB || ij;  // X(i, :) -= L(i, j) X(j, :) for i > j
-#pragma unroll
-      for (int c = 0; c <= CB; ++c) {
-        const double t = fma(-li[r], xj[c], x[r][c]);
-        x[r][c] = below ? t : x[r][c];
-      }
-    }
-  }
-}
-
-// NBK x NBK register blocks a lane, as wave_potrf_inv32 (h <= 8 NBK).
-template <bool EXACT, int NBK = 8>
-__device__ inline void wave_potrf_inv(double (*S)[NB + 1], double* xd, int o, int h, int lane,
-                                      const double* __restrict__ dg, int64_t col,
-                                      unsigned long long* __restrict__ fail, bool& bad) {
-  const int ti = lane & 7, tk = lane >> 3;
-  // the reference diagonal of every column, read once: the pivot test then costs a shuffle
-  const double dl = lane < h ? fabs(dg[lane]) : 0.0;
-  double a[NBK][NBK], x[NBK][NBK];
-#pragma unroll
-  for (int r = 0; r < NBK; ++r)
-#pragma unroll
-    for (int c = 0; c < NBK; ++c) {
-      const int i = ti + 8 * r, k = tk + 8 * c;
-      const double v = S[o + i][o + k];  // in bounds for every lane (o + 8 NBK <= NB)
-      a[r][c] = (i < h && k < h && i >= k) ? v : (i == k ? 1.0 : 0.0);
-      x[r][c] = i == k ? 1.0 : 0.0;
-    }
-  wpi_steps<0, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-  wpi_steps<1, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-  wpi_steps<2, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-  wpi_steps<3, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-  if constexpr (NBK > 4) {
-    wpi_steps<4, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-    wpi_steps<5, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-    wpi_steps<6, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-    wpi_steps<7, EXACT, NBK>(a, x, h, lane, dl, col, fail, bad);
-  }
-  // L below and on the diagonal, X above it (transposed), X's diagonal in xd; every lane
-  // stores to in-bounds addresses, the entries outside the h x h block are not written
-#pragma unroll
-  for (int r = 0; r < NBK; ++r)
-#pragma unroll
-    for (int c = 0; c < NBK; ++c) {
-      const int i = ti + 8 * r, k = tk + 8 * c;
-      if (i < h && k < h) {
-        if (i >= k) S[o + i][o + k] = a[r][c];
-        if (i > k) S[o + k][o + i] = x[r][c];
-        if (i == k) xd[o + i] = x[r][c];
-      }
-    }
-}
-
-// The same wave-local Cholesky and inverse in FP32 arithmetic, for the FP32-storage forms
-// (their diagonal blocks are FP32 work; the block's values are FP32 already). The steps are
-// those of wpi_steps, with the broadcast column zeroed outside the rows and columns a step
-// changes (L(i, j) for i <= j, L(k, j) for k <= j): the trailing updates then need no selects,
-// an update with a zero weight leaving its entry as it was. Entries above the diagonal of L's
-// diagonal register blocks take meaningless (finite) values and are never read or stored.
-// A pivot not above PIVOT_FP32 |A_jj| (or not finite) sets fb: the caller then factors the
-// whole block again in FP64, where the reference's pivot test decides.
-constexpr float PIVOT_FP32 = 1e-3f;
-
-__device__ __forceinline__ float readlane_f(float v, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-
-// NBK x NBK register blocks a lane (the wave covers blocks of up to 8 NBK columns): 8 for the
-// 64-column halves, 4 for 32-column quarters, whose steps touch a quarter of the registers.
-template <int CB, int NBK>
-__device__ __forceinline__ void wpi32_steps(float (&a)[NBK][NBK], float (&x)[NBK][NBK], int h, int lane, float dl,
-                                            bool& fb) {
-  const int ti = lane & 7, tk = lane >> 3;
-  for (int cc = 0; cc < 8; ++cc) {
-    const int j = 8 * CB + cc;
-    if (j >= h) return;
-    const float p = readlane_f(a[CB][CB], cc + 8 * cc);  // the pivot, on the step's dependent chain
-    const float a0 = readlane_f(dl, j);
-    fb = fb || !(p > PIVOT_FP32 * a0) || !(p < __builtin_huge_valf());
-    const float y = __builtin_amdgcn_rsqf(p);
-    const float rd = y * fmaf(-0.5f * p * y, y, 1.5f);  // 1 / sqrt(p), one Newton step
-    const float fc = tk == cc ? rd : 1.0f, fr = ti == cc ? rd : 1.0f;
-#pragma unroll
-    for (int r = CB; r < NBK; ++r) a[r][CB] *= fc;  // column j of L (the pivot becomes p rd = L(j, j))
-#pragma unroll
-    for (int c = 0; c <= CB; ++c) x[CB][c] *= fr;  // row j of X divided by L(j, j)
-    float li[NBK], lk[NBK], xj[NBK];
-#pragma unroll
-    for (int r = CB; r < NBK; ++r) li[r] = __shfl(a[r][CB], ti + 8 * cc);  // L(ti + 8r, j)
-#pragma unroll
-    for (int c = CB; c < NBK; ++c) lk[c] = __shfl(a[c][CB], tk + 8 * cc);  // L(tk + 8c, j)
-#pragma unroll
-    for (int c = 0; c <= CB; ++c) xj[c] = __shfl(x[CB][c], cc + 8 * tk);  // X(j, tk + 8c)
-    li[CB] = ti > cc ? li[CB] : 0.0f;
-    lk[CB] = tk > cc ? lk[CB] : 0.0f;
-#pragma unroll
-    for (int r = CB; r < NBK; ++r) {
-#pragma unroll
-      for (int c = CB; c <= r; ++c) a[r][c] = fmaf(-li[r], lk[c], a[r][c]);  // L(i, k) -= L(i, j) L(k, j)
-#pragma unroll
-      for (int c = 0; c <= CB; ++c) x[r][c] = fmaf(-li[r], xj[c], x[r][c]);  // X(i, :) -= L(i, j) X(j, :)
-    }
-  }
-}
-
-template <int NBK = 8>
-__device__ inline void wave_potrf_inv32(double (*S)[NB + 1], double* xd, int o, int h, int lane,
-                                        const double* __restrict__ dg, bool& fb) {
-  const int ti = lane & 7, tk = lane >> 3;
-  const float dl = lane < h ? (float)fabs(dg[lane]) : 0.0f;
-  float a[NBK][NBK], x[NBK][NBK];
-#pragma unroll
-  for (int r = 0; r < NBK; ++r)
-#pragma unroll
-    for (int c = 0; c < NBK; ++c) {
-      const int i = ti + 8 * r, k = tk + 8 * c;
-      const float v = (float)S[o + i][o + k];  // in bounds for every lane (o + 8 NBK <= NB)
-      a[r][c] = (i < h && k < h && i >= k) ? v : (i == k ? 1.0f : 0.0f);
-      x[r][c] = i == k ? 1.0f : 0.0f;
-    }
-  wpi32_steps<0, NBK>(a, x, h, lane, dl, fb);
-  wpi32_steps<1, NBK>(a, x, h, lane, dl, fb);
-  wpi32_steps<2, NBK>(a, x, h, lane, dl, fb);
-  wpi32_steps<3, NBK>(a, x, h, lane, dl, fb);
-  if constexpr (NBK > 4) {
-    wpi32_steps<4, NBK>(a, x, h, lane, dl, fb);
-    wpi32_steps<5, NBK>(a, x, h, lane, dl, fb);
-    wpi32_steps<6, NBK>(a, x, h, lane, dl, fb);
-    wpi32_steps<7, NBK>(a, x, h, lane, dl, fb);
-  }
-#pragma unroll
-  for (int r = 0; r < NBK; ++r)
-#pragma unroll
-    for (int c = 0; c < NBK; ++c) {
-      const int i = ti + 8 * r, k = tk + 8 * c;
-      if (i < h && k < h) {
-        if (i >= k) S[o + i][o + k] = a[r][c];
-        if (i > k) S[o + k][o + i] = x[r][c];
-        if (i == k) xd[o + i] = x[r][c];
-      }
-    }
-}
-
-// One wave's 16 x 16 tile of a product over k in [0, 32) on the FP64 MFMA:
-//   acc[v] = sum_k col(t, k) row(i, k),  i = lane % 16,  t = lane / 16 + 4 v
-// where col(t, k) and row(i, k) return in-bounds LDS values for t, i in [0, 16).
-template <class FC, class FR>
-__device__ __forceinline__ v4d tile16(int lane, FC col, FR row) {
-  const int r = lane & 15, q = lane >> 4;
-  v4d acc = {};
-#pragma unroll
-  for (int k0 = 0; k0 < 32; k0 += 4) acc = Mma<double>::step(col(r, k0 + q), row(r, k0 + q), acc);
-  return acc;
-}
-
-// The h x h block at S[o.., o..] (h <= 64) by the whole workgroup, with the layout the wave
-// functions leave: quarters of 32 columns, each factored and inverted inside one wave (4 x 4
-// register blocks a lane, whose steps cost under half the 64-column ones'), the products
-// between them on the FP64 MFMA, a 16 x 16 tile a wave (tile rows 16 (w % 2), columns
-// 16 (w / 2)), operands from LDS, triangular ones as 0/1 weights:
-//   L21 = A21 X11^T, A22 -= L21 L21^T, (L22, X22) in one wave, T = L21 X11, X21 = -X22 T.
-// T is 32 x 32 of LDS. Every thread calls it; it ends on a barrier.
-template <bool F32, bool EXACT>
-__device__ inline void half_potrf_inv(double (*S)[NB + 1], double* xd, double (*T)[33], int o, int h, int tid,
-                                      const double* __restrict__ dg, bool& fb, int64_t col,
-                                      unsigned long long* __restrict__ fail, bool& bad) {
-  const int lane = tid & 63, wave = tid >> 6;
-  const int h0 = min(32, h), h1 = h - h0, p = o + 32;
-  // one quarter's chain in wave 0: FP32 arithmetic (a small pivot sets fb), or FP64 with the
-  // reference's pivot test
-  auto chain = [&](int oq, int hq, int d) {
-    if constexpr (F32) wave_potrf_inv32<4>(S, xd, oq, hq, lane, dg + d, fb);
-    else wave_potrf_inv<EXACT, 4>(S, xd, oq, hq, lane, dg + d, col + d, fail, bad);
-  };
-  if (wave == 0) chain(o, h0, 0);
-  __syncthreads();
-  if (h1 <= 0) return;  // (uniform) h0 = 32 below
-  const int bi = 16 * (wave & 1), bt = 16 * (wave >> 1);  // the wave's tile
-  const int ri = lane & 15;
-  auto rowq = [&](int i) { return p + min(bi + i, h1 - 1); };  // a row of the second quarter, clamped
-  {  // L21(i, t) = sum_{k <= t} A21(i, k) X11(t, k); X11(t, k) = S[o + k][o + t] (t > k), xd[o + t]
-    const v4d acc = tile16(
-        lane,
-        [&](int t, int k) {
-          const int c = bt + t;
-          return S[o + k][o + c] * (c > k ? 1.0 : 0.0) + xd[o + c] * (c == k ? 1.0 : 0.0);
-        },
-        [&](int i, int k) { return S[rowq(i)][o + k]; });
-    __syncthreads();  // every A21 read before L21 is stored over it
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (bi + ri < h1) S[p + bi + ri][o + bt + (lane >> 4) + 4 * v] = acc[v];
-  }
-  __syncthreads();
-  if (bt <= bi) {  // A22(i, j) -= sum_k L21(i, k) L21(j, k), j <= i (reads the left quarter, writes the right)
-    const v4d acc = tile16(
-        lane, [&](int t, int k) { return S[p + min(bt + t, h1 - 1)][o + k]; }, [&](int i, int k) { return S[rowq(i)][o + k]; });
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int i = bi + ri, j = bt + (lane >> 4) + 4 * v;
-      if (i < h1 && j <= i) S[p + i][p + j] -= acc[v];
-    }
-  }
-  __syncthreads();
-  if (wave == 0) chain(p, h1, 32);
-  {  // T(i, c) = sum_{k >= c} L21(i, k) X11(k, c); X11(k, c) = S[o + c][o + k] (k > c), xd[o + c]
-    const v4d acc = tile16(
-        lane,
-        [&](int t, int k) {
-          const int c = bt + t;
-          return S[o + c][o + k] * (k > c ? 1.0 : 0.0) + xd[o + c] * (k == c ? 1.0 : 0.0);
-        },
-        [&](int i, int k) { return S[rowq(i)][o + k]; });
-#pragma unroll
-    for (int v = 0; v < 4; ++v) T[bi + ri][bt + (lane >> 4) + 4 * v] = acc[v];
-  }
-  __syncthreads();  // T, and the second quarter's factor and inverse, done
-  {  // X21(i, c) = -sum_{k <= i} X22(i, k) T(k, c); X22(i, k) = S[p + k][p + i] (i > k), xd[p + i];
-     // stored at S[o + c][p + i]. T's rows past h1 hold finite values (clamped rows) times 0
-    const v4d acc = tile16(
-        lane, [&](int t, int k) { return T[k][bt + t]; },
-        [&](int i, int k) {
-          const int ii = bi + i;
-          return S[p + k][p + ii] * (ii > k ? 1.0 : 0.0) + xd[p + ii] * (ii == k ? 1.0 : 0.0);
-        });
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (bi + ri < h1) S[o + bt + (lane >> 4) + 4 * v][p + bi + ri] = -acc[v];
-  }
-  __syncthreads();
-}
-
-// One wave's 64 x 16 strip of a product over k in [0, 64) on the FP64 MFMA:
-//   acc[ib][v] += sum_k col(t, k) row(i, k),  i = 16 ib + lane % 16,  t = (lane / 16) + 4 v
-// where col(r, k) and row(i, k) return in-bounds LDS values (col's r is the strip column in
-// [0, 16)). Each k-step reads one column value and four row values per lane for four MFMAs.
-template <class FC, class FR>
-__device__ __forceinline__ void strip64(v4d (&acc)[4], int lane, FC col, FR row) {
-  const int r = lane & 15, q = lane >> 4;
-#pragma unroll 4
-  for (int k0 = 0; k0 < 64; k0 += 4) {
-    const int k = k0 + q;
-    const double x = col(r, k);
-    double y[4];
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib) y[ib] = row(16 * ib + r, k);
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib) acc[ib] = Mma<double>::step(x, y[ib], acc[ib]);
-  }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256, 1) void k_potrf_blk(const Item* __restrict__ items, const FrontDev* __restrict__ fronts,
-                                                      T* __restrict__ L, const double* __restrict__ diag,
-                                                      unsigned long long* __restrict__ fail, T* __restrict__ Inv,
-                                                      __bf16* __restrict__ Lh, __bf16* __restrict__ Ll,
-                                                      const int32_t* __restrict__ fexp) {
-  constexpr int H = 64;
-  __shared__ double S[NB][NB + 1];
-  __shared__ double xd[NB];
-  __shared__ int redo;  // the FP32 attempt met a small pivot: factor again in FP64
-  __shared__ double Tq[32][33];  // the quarter products' scratch (half_potrf_inv)
-  const Item it = items[blockIdx.x];
-  const FrontDev F = fronts[it.f];
-  const int c0 = it.a, pw = min(NB, F.w - c0);
-  const int h0 = min(H, pw), h1 = pw - h0;
-  T* base = L + F.lpos + (int64_t)c0 * F.ld + c0;
-  const double* dg = diag + F.col0 + c0;
-  const int64_t col = (int64_t)F.col0 + c0;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rr = tid & (NB - 1), jp = tid >> 7;  // a thread's row, and which of every two columns
-  // Mixed form (Lh given): the block's scaled BF16 copies, from the same FP32 values as L (zero
-  // above the diagonal and past the block up to the next multiple of 32 columns), 8 columns of a
-  // row per 16-byte store. S holds the final L here (the products that follow overwrite L21).
-  auto copies = [&]() {
-    if (!Lh) return;
-    const float sc = ldexpf(1.0f, -fexp[it.f]);
-    const int ncp = (c0 + pw + 31) / 32 * 32 - c0;
-    for (int e = tid; e < pw * (ncp / 8); e += blockDim.x) {
-      const int r = e % pw, g = e / pw;
-      v8bf h, l;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int j = 8 * g + q;
-        const float x = (j <= r ? (float)(T)S[r][min(j, NB - 1)] : 0.0f) * sc;
-        h[q] = (__bf16)x;
-        l[q] = (__bf16)(x - (float)h[q]);
-      }
-      const int col = c0 + 8 * g;
-      const int64_t o = F.bpos + ((int64_t)(col / 32) * F.ld + c0 + r) * 32 + col % 32;
-      *(v8bf*)(Lh + o) = h;
-      *(v8bf*)(Ll + o) = l;
-    }
-  };
-  // the pw x pw square (its upper triangle is zeros in L, in bounds): 64 independent loads,
-  // through a buffer resource (the block spans far below 2 GiB of L): an entry outside the square
-  // takes the lane offset 2^31, past the resource's 2^31 - 1 bytes, and reads 0 from the buffer
-  // unit's range check, with no branch (a branch around each load made the compiler wait for
-  // each one in turn: 64 round trips, 28 us of a 73 us block).
-  // xd beyond the block's width is read by the products below with a 0 weight: it must hold a
-  // finite value, not what an earlier kernel left in LDS (a NaN there times 0 is a NaN)
-  const auto rs = raw_rsrc(base);
-  const uint32_t ldb = (uint32_t)F.ld * sizeof(T);
-  auto load = [&]() {
-    if (tid < NB) xd[tid] = 0.0;
-    T v[NB / 2];
-#pragma unroll
-    for (int q = 0; q < NB / 2; ++q) {
-      const int j = jp + 2 * q;
-      v[q] = buf_load<T>(rs, (rr < pw && j < pw) ? (uint32_t)(rr * sizeof(T)) : 0x80000000u, j * ldb);
-    }
-#pragma unroll
-    for (int q = 0; q < NB / 2; ++q) S[rr][jp + 2 * q] = (double)v[q];
-  };
-  // each wave: strip columns t0 + [0, 16) of a 64 x 64 product, rows 16 ib + lane % 16
-  const int r = lane & 15, q = lane >> 4, t0 = 16 * wave;
-  // L11 and X11; for a wide panel then L21 = A21 X11^T, A22 -= L21 L21^T, L22 and X22, each half
-  // by the whole workgroup in 32-column quarters. F32: the wave steps in FP32 arithmetic (a
-  // small pivot sets redo); otherwise FP64 with the reference's pivot test.
-  bool bad = false;
-  auto factor = [&](auto f32) {
-    constexpr bool F32 = decltype(f32)::value;
-    bool fb = false;
-    half_potrf_inv<F32, sizeof(T) == 8>(S, xd, Tq, 0, h0, tid, dg, fb, col, fail, bad);
-    __syncthreads();
-    if (h1 > 0) {
-      {  // L21 = A21 X11^T: L21(i, t) = sum_{k <= t} A21(i, k) X11(t, k), X11(t, k) = S[k][t] (t > k)
-        v4d acc[4] = {};
-        strip64(
-            acc, lane,
-            [&](int c, int k) {  // 0/1 weights, not selects: the loads stay unconditional
-              const int t = t0 + c;
-              return S[k][t] * (t > k ? 1.0 : 0.0) + xd[k] * (t == k ? 1.0 : 0.0);
-            },
-            [&](int i, int k) { return S[h0 + min(i, h1 - 1)][k]; });
-        __syncthreads();  // every A21 read before L21 is stored over it
-#pragma unroll
-        for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int i = 16 * ib + r;
-            if (i < h1) S[h0 + i][t0 + q + 4 * v] = acc[ib][v];
-          }
-      }
-      __syncthreads();
-      {  // A22 -= L21 L21^T over the lower triangle (reads the left half, writes the right)
-        v4d acc[4] = {};
-        strip64(
-            acc, lane, [&](int c, int k) { return S[h0 + min(t0 + c, h1 - 1)][k]; },
-            [&](int i, int k) { return S[h0 + min(i, h1 - 1)][k]; });
-#pragma unroll
-        for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int i = 16 * ib + r, j = t0 + q + 4 * v;
-            if (i < h1 && j <= i) S[h0 + i][h0 + j] -= acc[ib][v];
-          }
-      }
-      __syncthreads();
-      half_potrf_inv<F32, sizeof(T) == 8>(S, xd, Tq, h0, h1, tid, dg + h0, fb, col + h0, fail, bad);
-    }
-    if constexpr (F32) {
-      if (wave == 0 && lane == 0) redo = fb ? 1 : 0;
-    }
-    __syncthreads();
-  };
-  load();
-  __syncthreads();
-  if constexpr (sizeof(T) == 4) {
-    factor(std::true_type{});
-    if (redo) {  // uniform: read by every thread after the barrier that ends factor()
-      __syncthreads();  // every thread has read redo before S is loaded again
-      load();
-      __syncthreads();
-      factor(std::false_type{});
-    }
-  } else {
-    factor(std::false_type{});
-  }
-  // L is final: write it out (reads first, then stores), and its copies
-  {
-    T v[NB / 2];
-#pragma unroll
-    for (int qq = 0; qq < NB / 2; ++qq) v[qq] = (T)S[rr][jp + 2 * qq];
-#pragma unroll
-    for (int qq = 0; qq < NB / 2; ++qq) {
-      const int j = jp + 2 * qq;
-      if (rr < pw && j <= rr) base[(int64_t)j * F.ld + rr] = v[qq];
-    }
-  }
-  copies();
-  if (h1 > 0) {
-    {  // T = L21 X11: T(i, t) = sum_{k >= t} L21(i, k) X11(k, t), X11(k, t) = S[t][k] (k > t)
-      v4d acc[4] = {};
-      strip64(
-          acc, lane,
-          [&](int c, int k) {
-            const int t = t0 + c;
-            return S[t][k] * (k > t ? 1.0 : 0.0) + xd[k] * (k == t ? 1.0 : 0.0);
-          },
-          [&](int i, int k) { return S[h0 + min(i, h1 - 1)][k]; });
-      __syncthreads();  // L21 written out and read
-#pragma unroll
-      for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * ib + r;
-          if (i < h1) S[h0 + i][t0 + q + 4 * v] = acc[ib][v];  // T over L21
-        }
-    }
-    __syncthreads();
-    {  // X21 = -X22 T, stored at S[t][h0 + ii]: X22(ii, k) = S[h0 + k][h0 + ii] (ii > k), T(k, t) = S[h0 + k][t]
-      v4d acc[4] = {};
-      strip64(
-          acc, lane, [&](int c, int k) { return S[h0 + k][t0 + c]; },
-          [&](int ii, int k) {
-            return S[h0 + k][h0 + ii] * (ii > k ? 1.0 : 0.0) + xd[h0 + k] * (ii == k ? 1.0 : 0.0);
-          });
-#pragma unroll
-      for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int ii = 16 * ib + r;
-          if (ii < h1) S[t0 + q + 4 * v][h0 + ii] = -acc[ib][v];
-        }
-    }
-  }
-  __syncthreads();
-  {  // the inverse, column-major with ld = pw, zeros above the diagonal: reads, then stores
-    T* inv = Inv + F.inv0 + (int64_t)(c0 / NB) * NB * NB;
-    T v[NB / 2];
-    const double xr = xd[rr];
-#pragma unroll
-    for (int q = 0; q < NB / 2; ++q) {
-      const int j = jp + 2 * q;
-      v[q] = (T)(S[j][rr] * (rr > j ? 1.0 : 0.0) + xr * (rr == j ? 1.0 : 0.0));
-    }
-#pragma unroll
-    for (int q = 0; q < NB / 2; ++q) {
-      const int j = jp + 2 * q;
-      if (rr < pw && j < pw) inv[(int64_t)j * pw + rr] = v[q];
-    }
-  }
-}
-
 }  // namespace fc

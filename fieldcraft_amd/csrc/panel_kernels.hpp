@@ -1,7 +1,8 @@
 // A panel's diagonal block and the rows below it on the matrix cores (gfx950).
 //
 // diag_potrf_inv factors and inverts a diagonal block of up to 128 columns in LDS by one
-// workgroup, for k_small_fronts; block_substitute solves sixteen rows a wave against a factored block without leaving the wave's registers.
+// workgroup (k_potrf_blk: a panel's; k_small_fronts: a small front's); substitute_block solves
+// sixteen rows a wave against a factored block without leaving the wave's registers.
 #pragma once
 
 #include "gemm_kernels.hpp"
@@ -9,6 +10,15 @@
 namespace fc {
 
 constexpr int DB = 16;  // columns of a diagonal-block step: one MFMA tile
+constexpr double PIVOT_TOL = 1e-10;  // cholesky.rs:48
+
+// A double from one lane (uniform index) to the whole wave, by scalar reads of its halves.
+__device__ __forceinline__ double readlane_d(double v, int l) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, l);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
 
 // d = sqrt(p) and rd = 1 / sqrt(p), both to within a rounding or so: the hardware's estimate, one
 // coupled Newton step on (sqrt p, 1 / (2 sqrt p)), then each corrected by its own residual.
@@ -27,8 +37,11 @@ __device__ __forceinline__ void root_pair(double p, double& d, double& rd) {
 // reference's pivot test (cholesky.rs:1161) and inverted, in FP64 (EXACT: the quotients by the
 // pivot's root rounded as divisions, for FP64 storage). On entry S holds A in its lower
 // triangle over the 16 nb x 16 nb square (nb = ceil(h / 16)), zeros above it, and an identity in
-// the rows and columns past h; on return S[i][j] = L(i, j) for i >= j, S[k][i] = Linv(i, k) for
-// i > k and xd[i] = Linv(i, i). IB is 16 x 17 of LDS. NW waves call it; it ends on a barrier.
+// the rows and columns past h; on return S[i][j] = L(i, j) for i >= j, the inverse's diagonal
+// blocks are X[b] (transposed: X[b][c][r] = Linv(16 b + r, 16 b + c), zeros for r < c) and its other
+// blocks lie transposed above the diagonal blocks of S, S[k][i] = Linv(i, k) (diag_inv reads an
+// entry). The entries of S above the diagonal inside a diagonal block are left undefined. One wave
+// per 16 rows of NMAX calls it together; it ends on a barrier.
 //
 // A block of 128 columns is a chain of 128 dependent pivots, so what sets its time is the
 // latency of a step. Each step of 16 columns is taken by every wave on its own copy of the 16 x 16
@@ -39,28 +52,31 @@ __device__ __forceinline__ void root_pair(double p, double& d, double& rd) {
 // LDS round trip and no barrier inside a step). Row c of the identity is nonzero from column c
 // on, so its entries live in the upper triangle of S and each step has 16 nb rows to take. The
 // trailing update S(r, j) -= P(r) L(j)^T (rows below, and identity rows already started) goes
-// through the 16x16x4 MFMA, a tile a wave, NT tiles of a wave in flight at once.
-template <int NMAX, int NW, bool EXACT>
-__device__ inline void diag_potrf_inv(double (*S)[NMAX + 1], double* xd, double (*IB)[DB + 1], int h, int tid,
+// through the 16x16x4 MFMA, row block r by wave r. Measured, a 128-column block: 90 us with a wave's
+// 8 x 8 lane grid passing columns through LDS shuffles on 32-column quarters, and products between
+// the quarters (FP32 arithmetic: 60 us); 38 us in this form, the pivots' chain 12 us of it, the tiles 9.
+template <int NMAX>
+using DiagX = double[NMAX / DB][DB][DB + 1];
+
+template <int NMAX, bool EXACT>
+__device__ inline void diag_potrf_inv(double (*S)[NMAX + 1], DiagX<NMAX>& X, int h, int tid,
                                       const double* __restrict__ dg, int64_t col,
                                       unsigned long long* __restrict__ fail) {
   constexpr int ROWS = 64 - DB;  // rows a wave takes beside the pivot block
-  static_assert(NW * ROWS >= NMAX, "a step's rows fit the workgroup's waves");
-  constexpr int NT = 3;
-  const int lane = tid & 63, wave = tid >> 6;
+  static_assert(NMAX / DB * ROWS >= NMAX, "a step's rows fit the workgroup's waves");
+  const int lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
   const int nb = (h + DB - 1) / DB;
   for (int kb = 0; kb < nb; ++kb) {
     const int c0 = DB * kb;
     // slot 0..15: the identity's rows c0 ..; then the block's other rows in order
     const int slot = wave * ROWS + lane - DB;
     const bool piv = lane < DB, ident = !piv && slot < DB, act = !piv && slot < DB * nb;
-    const int row = piv ? c0 + lane : (slot - DB < c0 ? slot - DB : slot);  // (unused for the identity)
+    const int row = (piv || ident || !act) ? c0 + (piv ? lane : 0) : (slot - DB < c0 ? slot - DB : slot);
     const bool work = wave * ROWS < DB * nb;  // uniform
     double a[DB];
     if (work) {
-      const double* src = S[(piv || (act && !ident)) ? row : c0];
 #pragma unroll
-      for (int t = 0; t < DB; ++t) a[t] = src[c0 + t];
+      for (int t = 0; t < DB; ++t) a[t] = S[row][c0 + t];
       if (ident)
 #pragma unroll
         for (int t = 0; t < DB; ++t) a[t] = t == slot ? 1.0 : 0.0;
@@ -68,7 +84,7 @@ __device__ inline void diag_potrf_inv(double (*S)[NMAX + 1], double* xd, double 
     const double dl = (lane < DB && c0 + lane < h) ? fabs(dg[c0 + lane]) : 0.0;
     __syncthreads();  // every copy of the pivot block read before it is overwritten
     if (work) {
-double pv = 0.0;  // lane j: pivot j
+      double pv = 0.0;  // lane j: pivot j
       double p = readlane_d(a[0], 0), d, rd;
       root_pair(p, d, rd);
 #pragma unroll
@@ -91,54 +107,124 @@ double pv = 0.0;  // lane j: pivot j
       }
       if (wave == 0 && lane < DB && c0 + lane < h && (!(pv > PIVOT_TOL * dl) || !isfinite(pv)))
         atomicMin(fail, (unsigned long long)(col + c0 + lane));
-      if (ident) {
+      if (act || (piv && wave == 0)) {
+        double* dst = ident ? X[kb][slot] : &S[row][c0];
 #pragma unroll
-        for (int t = 0; t < DB; ++t) {
-          IB[slot][t] = a[t];
-          if (t > slot) S[c0 + slot][c0 + t] = a[t];
-          if (t == slot) xd[c0 + slot] = a[t];
-        }
-      } else if (act || (piv && wave == 0)) {
-#pragma unroll
-        for (int t = 0; t < DB; ++t)
-          if (!piv || t <= lane) S[row][c0 + t] = a[t];
+        for (int t = 0; t < DB; ++t) dst[t] = a[t];
       }
     }
     __syncthreads();
-    // tiles (r, j), j > kb: rows r >= j (below) and r <= kb (the identity's)
-    const int nj = nb - 1 - kb;
-    const int tiles = nj * (nj + 1) / 2 + nj * (kb + 1);
-    for (int t0 = wave; t0 < tiles; t0 += NW * NT) {
-      int rb[NT], jb[NT];
-      v4d acc[NT];
+    // row block `wave`: every column block after kb up to its own (below), or all (the identity's)
+    const int hi = wave > kb ? min(wave, nb - 1) : nb - 1;
+    if (wave < nb) {
+      const double* src = wave == kb ? X[kb][r] : &S[DB * wave + r][c0];
+      double fi[4];
 #pragma unroll
-      for (int q = 0; q < NT; ++q) {
-        int t = min(t0 + NW * q, tiles - 1), j = 0;
-        while (t >= (kb + 1) + (nj - j)) t -= (kb + 1) + (nj - j), ++j;  // column kb + 1 + j
-        jb[q] = kb + 1 + j;
-        rb[q] = t <= kb ? t : jb[q] + t - (kb + 1);
-        acc[q] = v4d{0, 0, 0, 0};
+      for (int s = 0; s < 4; ++s) fi[s] = -src[4 * s + g];
+      for (int jb = kb + 1; jb <= hi; ++jb) {
+        double* out = &S[DB * wave + r][DB * jb + g];
+        double fj[4];
+        v4d acc;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) fj[s] = S[DB * jb + r][c0 + 4 * s + g];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[v] = out[4 * v];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = Mma<double>::step(fj[s], fi[s], acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out[4 * v] = acc[v];
       }
-      const int r = lane & 15, g = lane >> 4;
-      double fj[NT][4], fi[NT][4];
-#pragma unroll
-      for (int q = 0; q < NT; ++q)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          fj[q][s] = S[DB * jb[q] + r][c0 + 4 * s + g];
-          fi[q][s] = rb[q] == kb ? IB[r][4 * s + g] : S[DB * rb[q] + r][c0 + 4 * s + g];
-        }
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int q = 0; q < NT; ++q) acc[q] = Mma<double>::step(fj[q][s], fi[q][s], acc[q]);
-#pragma unroll
-      for (int q = 0; q < NT; ++q)
-        if (t0 + NW * q < tiles)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) S[DB * rb[q] + r][DB * jb[q] + g + 4 * v] -= acc[q][v];
     }
     __syncthreads();
+  }
+}
+
+// Linv(i, j), i >= j, of a block diag_potrf_inv has left.
+template <int NMAX>
+__device__ __forceinline__ double diag_inv(const double (*S)[NMAX + 1], const DiagX<NMAX>& X, int i, int j) {
+  return i / DB == j / DB ? X[i / DB][j % DB][i % DB] : S[j][i];
+}
+
+// The diagonal block of a panel (any width up to NB; item: f, a = c0): factored with the
+// reference's pivot test (cholesky.rs:1146-1171: a pivot not above 1e-10 |A_jj|, or not finite,
+// fails the column) and inverted, in FP64 arithmetic whatever the storage. L11 goes over the
+// block's lower triangle in L, Linv (pw x pw, column-major, zeros above the diagonal) to the
+// panel's slot of Inv (F.inv0 + (c0 / NB) NB^2). One workgroup a block: the chain of pivots bounds
+// it (diag_potrf_inv), so the loads and stores around it are made in one batch each.
+constexpr int POTRF_THREADS = 512;
+template <typename T>
+__global__ __launch_bounds__(POTRF_THREADS, 1) void k_potrf_blk(const Item* __restrict__ items,
+                                                                const FrontDev* __restrict__ fronts, T* __restrict__ L,
+                                                                const double* __restrict__ diag,
+                                                                unsigned long long* __restrict__ fail, T* __restrict__ Inv,
+                                                                __bf16* __restrict__ Lh, __bf16* __restrict__ Ll,
+                                                                const int32_t* __restrict__ fexp) {
+  static_assert(POTRF_THREADS == 64 * (NB / DB), "a wave a row block");
+  __shared__ double S[NB][NB + 1];
+  __shared__ DiagX<NB> X;
+  constexpr int CQ = POTRF_THREADS / NB, Q = NB / CQ;  // thread: one row, every CQ-th column
+  const Item it = items[blockIdx.x];
+  const FrontDev F = fronts[it.f];
+  const int c0 = it.a, pw = min(NB, F.w - c0);
+  T* base = L + F.lpos + (int64_t)c0 * F.ld + c0;
+  const int tid = threadIdx.x, rr = tid & (NB - 1), jp = tid / NB;
+  {
+    // the lower triangle through a buffer resource (the block spans far below 2 GiB of L): an entry
+    // outside it takes the lane offset 2^31, past the resource's 2^31 - 1 bytes, and reads 0 from
+    // the buffer unit's range check, with no branch around the load
+    const auto rs = raw_rsrc(base);
+    const uint32_t ldb = (uint32_t)F.ld * sizeof(T);
+    T v[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int j = jp + CQ * q;
+      v[q] = buf_load<T>(rs, (rr < pw && j <= rr) ? (uint32_t)(rr * sizeof(T)) : 0x80000000u, j * ldb);
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int j = jp + CQ * q;
+      S[rr][j] = (rr == j && rr >= pw) ? 1.0 : (double)v[q];
+    }
+  }
+  __syncthreads();
+  diag_potrf_inv<NB, sizeof(T) == 8>(S, X, pw, tid, diag + F.col0 + c0, (int64_t)F.col0 + c0, fail);
+  {
+    T* inv = Inv + F.inv0 + (int64_t)(c0 / NB) * NB * NB;
+    T v[Q], x[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int j = jp + CQ * q;
+      v[q] = (T)S[rr][j];
+      x[q] = (rr >= j && rr < pw) ? (T)diag_inv<NB>(S, X, rr, j) : T(0);
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int j = jp + CQ * q;
+      if (rr < pw && j <= rr) base[(int64_t)j * F.ld + rr] = v[q];
+      if (rr < pw && j < pw) inv[(int64_t)j * pw + rr] = x[q];
+    }
+  }
+  // Mixed form (Lh given): the block's scaled BF16 copies, from the same FP32 values as L (zero
+  // above the diagonal and past the block up to the next multiple of 32 columns), 8 columns of a
+  // row per 16-byte store.
+  if (Lh) {
+    const float sc = ldexpf(1.0f, -fexp[it.f]);
+    const int ncp = (c0 + pw + 31) / 32 * 32 - c0;
+    for (int e = tid; e < pw * (ncp / 8); e += POTRF_THREADS) {
+      const int r = e % pw, g = e / pw;
+      v8bf h, l;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int j = 8 * g + q;
+        const float x = (j <= r ? (float)(T)S[r][min(j, NB - 1)] : 0.0f) * sc;
+        h[q] = (__bf16)x;
+        l[q] = (__bf16)(x - (float)h[q]);
+      }
+      const int col = c0 + 8 * g;
+      const int64_t o = F.bpos + ((int64_t)(col / 32) * F.ld + c0 + r) * 32 + col % 32;
+      *(v8bf*)(Lh + o) = h;
+      *(v8bf*)(Ll + o) = l;
+    }
   }
 }
 
@@ -147,31 +233,28 @@ double pv = 0.0;  // lane j: pivot j
 // x[k] holds B_k on entry and X_k on return, in the MFMA's output layout (entry v of a lane: row
 // lane % 16, column 16 k + row(lane, v)). That layout is also the layout of the next product's
 // row operand when the products sum their 16 columns in the order row(lane, s), so no value moves
-// between lanes. Lop(k, j, s), Xop(k, s) and Dop(k, s) return the lane's column operand: entry
-// (lane % 16, row(lane, s)) of L_kj, L_kk^-1 and L_kk. REFINE corrects each X_k once against L_kk
+// between lanes. Lop(j, s), Xop(s) and Dop(s) return the lane's column operand: entry
+// (lane % 16, row(lane, s)) of L_kj, L_kk^-1 and L_kk (k a constant of the unrolled caller). REFINE corrects each X_k once against L_kk
 // (a product with an explicit inverse alone is not backward stable).
-template <typename M, int NBK, bool REFINE, class FL, class FX, class FD>
-__device__ __forceinline__ void block_substitute(typename Mma<M>::acc_t (&x)[NBK], int nb, FL Lop, FX Xop, FD Dop) {
+template <typename M, bool REFINE, int NBK, class FL, class FX, class FD>
+__device__ __forceinline__ void substitute_block(typename Mma<M>::acc_t (&x)[NBK], int k, FL Lop, FX Xop, FD Dop) {
   typedef typename Mma<M>::acc_t acc_t;
+  acc_t b = x[k];
 #pragma unroll
-  for (int k = 0; k < NBK; ++k) {
-    if (k >= nb) break;
-    acc_t b = x[k];
+  for (int j = 0; j < NBK; ++j)
+    if (j < k)
 #pragma unroll
-    for (int j = 0; j < k; ++j)
+      for (int s = 0; s < 4; ++s) b = Mma<M>::step(-Lop(j, s), x[j][s], b);
+  acc_t y = {0, 0, 0, 0};
 #pragma unroll
-      for (int s = 0; s < 4; ++s) b = Mma<M>::step(-Lop(k, j, s), x[j][s], b);
-    acc_t y = {0, 0, 0, 0};
+  for (int s = 0; s < 4; ++s) y = Mma<M>::step(Xop(s), b[s], y);
+  if constexpr (REFINE) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) y = Mma<M>::step(Xop(k, s), b[s], y);
-    if constexpr (REFINE) {
+    for (int s = 0; s < 4; ++s) b = Mma<M>::step(-Dop(s), y[s], b);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) b = Mma<M>::step(-Dop(k, s), y[s], b);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) y = Mma<M>::step(Xop(k, s), b[s], y);
-    }
-    x[k] = y;
+    for (int s = 0; s < 4; ++s) y = Mma<M>::step(Xop(s), b[s], y);
   }
+  x[k] = y;
 }
 
 }  // namespace fc

@@ -1164,7 +1164,7 @@ void enqueue_factor(fc_factor* F, const double* dval, i64 nnz, hipStream_t st, b
         fc::k_reduce_parts<T><<<dim3(l.count * fc::RSPLIT), b, 0, ls>>>(P.ritems + l.item0, L, U, Part);
         break;
       case fc::K_POTRF:
-        fc::k_potrf_blk<T><<<g, dim3(256), 0, ls>>>(it, P.fronts, L, F->diag, F->fail, Inv, Lh, Ll, fexp);
+        fc::k_potrf_blk<T><<<g, dim3(fc::POTRF_THREADS), 0, ls>>>(it, P.fronts, L, F->diag, F->fail, Inv, Lh, Ll, fexp);
         break;
       case fc::K_SMALL:
         fc::k_small_fronts<T><<<g, b, 0, ls>>>(it, P.fronts, L, U, F->diag, F->fail, Inv);

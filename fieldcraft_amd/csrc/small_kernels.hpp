@@ -9,7 +9,7 @@
 //   1. its diagonal block, factored and inverted in LDS (diag_potrf_inv), L11 and the inverse
 //      written out;
 //   2. the rows below by block substitution on the matrix cores, sixteen rows a wave
-//      (block_substitute; the FP64 factor refines each block once, as the tiled path does);
+//      (substitute_block; the FP64 factor refines each block once, as the tiled path does);
 //   3. its update matrix U = -L21 L21^T (lower triangle), 32 x 32 tiles a wave on the matrix cores.
 // The values end where the tiled path puts them (L, Inv, U); the FP32-storage forms write no
 // BF16 copies for them, since no product of the tiled path reads a small front.
@@ -36,8 +36,7 @@ __global__ __launch_bounds__(256, 2) void k_small_fronts(const Item* __restrict_
                                                          T* __restrict__ U, const double* __restrict__ diag,
                                                          unsigned long long* __restrict__ fail, T* __restrict__ Inv) {
   __shared__ double S[SMALL_W][SMALL_W + 1];
-  __shared__ double xd[SMALL_W];
-  __shared__ double IB[DB][DB + 1];
+  __shared__ DiagX<SMALL_W> X;
   constexpr uint32_t OUT = 0x80000000u;  // a lane offset past a buffer resource: reads 0, stores nothing
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const FrontDev F = fronts[items[blockIdx.x].f];
@@ -62,12 +61,12 @@ __global__ __launch_bounds__(256, 2) void k_small_fronts(const Item* __restrict_
     }
   }
   __syncthreads();
-  diag_potrf_inv<SMALL_W, 4, sizeof(T) == 8>(S, xd, IB, w, tid, diag + F.col0, F.col0, fail);
+  diag_potrf_inv<SMALL_W, sizeof(T) == 8>(S, X, w, tid, diag + F.col0, F.col0, fail);
   // L11 out, and the inverse (column-major, ld = w, zeros above the diagonal)
   for (int e = tid; e < w * w; e += blockDim.x) {
     const int i = e % w, j = e / w;
     if (j <= i) base[(int64_t)j * F.ld + i] = (T)S[i][j];
-    Inv[F.inv0 + (int64_t)j * w + i] = (T)(i > j ? S[j][i] : (i == j ? xd[i] : 0.0));
+    Inv[F.inv0 + (int64_t)j * w + i] = i >= j ? (T)diag_inv<SMALL_W>(S, X, i, j) : T(0);
   }
   // 2. the rows below, sixteen a wave: entry v of x[k] is row i, column 16 k + lane / 16 + 4 v
   const int r = lane & 15, g = lane >> 4;
@@ -84,18 +83,18 @@ __global__ __launch_bounds__(256, 2) void k_small_fronts(const Item* __restrict_
     for (int k = 0; k < NBK; ++k)
 #pragma unroll
       for (int v = 0; v < 4; ++v) x[k][v] = (double)b[k][v];
-    block_substitute<double, NBK, sizeof(T) == 8>(
-        x, nb, [&](int k, int j, int s) { return S[16 * k + r][16 * j + 4 * s + g]; },
-        [&](int k, int s) {  // Linv(r, c) of the block: S[c][r] below the diagonal, xd on it
-          const int c = 4 * s + g;
-          const double v = S[16 * k + (c < r ? c : r)][16 * k + r];
-          return c < r ? v : (c == r ? xd[16 * k + r] : 0.0);
-        },
-        [&](int k, int s) {
-          const int c = 4 * s + g;
-          const double v = S[16 * k + r][16 * k + c];
-          return c <= r ? v : 0.0;
-        });
+#pragma unroll
+    for (int k = 0; k < NBK; ++k) {
+      if (k >= nb) break;
+      substitute_block<double, sizeof(T) == 8>(
+          x, k, [&](int j, int s) { return S[16 * k + r][16 * j + 4 * s + g]; },
+          [&](int s) { return X[k][4 * s + g][r]; },
+          [&](int s) {
+            const int c = 4 * s + g;
+            const double v = S[16 * k + r][16 * k + c];
+            return c <= r ? v : 0.0;
+          });
+    }
 #pragma unroll
     for (int k = 0; k < NBK; ++k)
 #pragma unroll
