@@ -2,10 +2,8 @@
 //
 // Every GEMM-shaped step of the numeric phase is one item of one kernel, k_gemm:
 //   panel update   L[r.., c0..c1) -= L[r.., 0..c0) L[c0..c1, 0..c0)^T      (G_SUB)
-//   rows below     L[r.., c0..c1)  = L[r.., c0..c1) Linv^T                   (G_SET, in place)
 //   update matrix  U[i.., j..)     = -L[W+i.., 0..W) L[W+j.., 0..W)^T        (G_NEG)
-// where Linv is the inverse of the panel's factored diagonal block (k_potrf_blk). A launch
-// with few output tiles is split along k: each piece writes its partial tile (G_PART) and
+// (the rows below a panel's diagonal block are panel_kernels.hpp's). A launch with few output tiles is split along k: each piece writes its partial tile (G_PART) and
 // k_reduce_parts adds the pieces in a fixed order, so results do not depend on scheduling.
 //
 // Tile: 128 x 128 per workgroup of 4 waves, each wave a 64 x 64 quarter as 4 x 4 blocks of the
@@ -26,8 +24,8 @@ constexpr int GB = 128;  // tile edge
 constexpr int GK = 16;   // k per LDS stage
 constexpr int NB = 128;  // panel width of the factorization (columns of a diagonal block)
 
-enum GemmMode : int32_t { G_SUB = 0, G_NEG = 1, G_SET = 2, G_PART = 3, G_ADD = 4 };
-enum GemmSrc : int8_t { S_L = 0, S_U = 1, S_INV = 2, S_PART = 3, S_W = 4 };
+enum GemmMode : int32_t { G_SUB = 0, G_NEG = 1, G_PART = 2 };
+enum GemmSrc : int8_t { S_L = 0, S_U = 1, S_PART = 2 };
 
 struct GemmItem {
   int64_t a, b, c;        // element offsets: A(i, k) = A[a + k lda + i], B(j, k), C(i, j) = C[c + j ldc + i]
@@ -35,7 +33,7 @@ struct GemmItem {
   int32_t m, n, k;        // rows of C (and A), columns of C (rows of B), depth
   int32_t mode;           // GemmMode
   int32_t diag;           // store C(i, j) only when i - j + diag >= 0
-  int8_t asrc, bsrc, csrc, pad0;
+  int8_t csrc, pad0, pad1, pad2;
   int32_t front;          // the front both operands come from (its scale in the mixed form)
 };
 static_assert(sizeof(GemmItem) == 64, "GemmItem layout");
@@ -69,21 +67,14 @@ struct Mma<float> {
   static __device__ __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
-// SPLIT (FP32, in-place rows-below products of the mixed form): the epilogue also writes the
-// result's scaled BF16 copies (see k_gemm_b16), so a finished panel needs no pass of its own.
-template <typename T, bool SPLIT = false>
-__global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ items, T* L, T* U, T* Inv, T* Part, T* W,
-                                                 const FrontDev* __restrict__ fronts, __bf16* __restrict__ Lh,
-                                                 __bf16* __restrict__ Ll, const int32_t* __restrict__ fexp) {
+template <typename T>
+__global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ items, T* L, T* U, T* Part) {
   constexpr int PAD = 4;
   __shared__ T As[2][GK][GB + PAD];
   __shared__ T Bs[2][GK][GB + PAD];
   const GemmItem it = items[blockIdx.x];
-  auto base = [&](int8_t src) {
-    return src == S_L ? L : (src == S_U ? U : (src == S_INV ? Inv : (src == S_W ? W : Part)));
-  };
-  const T* __restrict__ A = base(it.asrc) + it.a;
-  const T* __restrict__ B = base(it.bsrc) + it.b;
+  const T* __restrict__ A = L + it.a;
+  const T* __restrict__ B = L + it.b;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;
   const int lrow = tid & (GB - 1), lk = tid >> 7;  // loader: one row, every other k
@@ -148,18 +139,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ it
         }
     return;
   }
-  T* C = base(it.csrc) + it.c;
-  // By row blocks: G_SUB and G_ADD read the block's 16 old values first, every load in flight at
+  T* C = (it.csrc == S_L ? L : U) + it.c;
+  // By row blocks: G_SUB reads the block's 16 old values first, every load in flight at
   // once, through a buffer resource (a tile spans far below 2 GiB of its array; an entry outside
   // the tile reads 0 from the range check and is not stored). An update and its load in one
   // branch made the compiler wait for each load in turn: 64 round trips a tile.
-  const bool rmw = it.mode == G_SUB || it.mode == G_ADD;
   const auto rc = raw_rsrc(C);
   const uint32_t ldcb = (uint32_t)it.ldc * sizeof(T);
 #pragma unroll
   for (int bi = 0; bi < 4; ++bi) {
     T old[4][4] = {};
-    if (rmw) {
+    if (it.mode == G_SUB) {
 #pragma unroll
       for (int bj = 0; bj < 4; ++bj)
 #pragma unroll
@@ -176,69 +166,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ it
         const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<T>::row(lane, v);
         if (i < it.m && j < it.n && i - j + it.diag >= 0) {
           const T x = acc[bi][bj][v];
-          C[(int64_t)j * it.ldc + i] =
-              it.mode == G_SUB ? old[bj][v] - x : (it.mode == G_ADD ? old[bj][v] + x : (it.mode == G_NEG ? -x : x));
+          C[(int64_t)j * it.ldc + i] = it.mode == G_SUB ? old[bj][v] - x : -x;
         }
       }
-  }
-  if constexpr (SPLIT) {
-    static_assert(sizeof(T) == 4, "copies of an FP32 result");
-    // a lane's four values of a block are consecutive columns of one row: one 8-byte store a
-    // copy. Columns from n up to the next multiple of 32 (the last panel of a front) are zeros
-    // (the product's B rows past n load as zeros).
-    const FrontDev F = fronts[it.front];
-    const float sc = ldexpf(1.0f, -fexp[it.front]);
-    const int64_t oc = it.c - F.lpos;
-    const int row0 = (int)(oc % F.ld), col0 = (int)(oc / F.ld);
-    const int ncp = (col0 + it.n + 31) / 32 * 32 - col0;
-#pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < 4; ++bj) {
-        const int i = wi + 16 * bi + il, j = wj + 16 * bj + 4 * (lane >> 4);
-        if (i < it.m && j < ncp) {
-          __bf16 h[4], l[4];
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float x = (float)acc[bi][bj][v] * sc;
-            h[v] = (__bf16)x;
-            l[v] = (__bf16)(x - (float)h[v]);
-          }
-          const int col = col0 + j;
-          const int64_t o = F.bpos + ((int64_t)(col / 32) * F.ld + row0 + i) * 32 + col % 32;
-          *(uint2*)(Lh + o) = *(const uint2*)h;
-          *(uint2*)(Ll + o) = *(const uint2*)l;
-        }
-      }
-  }
-}
-
-// A tile's entries C(i, j) = A(i, j) (i < m <= GB, j < n <= GB): the rows below a panel saved
-// before the product that overwrites them (the FP64 TRSM refines its result against them).
-// Wave v copies columns v, v + 4, ...; lane l rows l and l + 64 of each, so every wave load and
-// store covers 64 consecutive entries of one column. CB columns' loads are issued before any
-// store (rows and columns past the tile load its last entry, which is not stored).
-template <typename T>
-__global__ __launch_bounds__(256) void k_copy_tiles(const GemmItem* __restrict__ items, const T* __restrict__ L,
-                                                    T* __restrict__ W) {
-  constexpr int CB = 8;
-  static_assert(GB <= 128, "two rows a lane cover a tile's rows");
-  const GemmItem it = items[blockIdx.x];
-  const T* A = L + it.a;
-  T* C = W + it.c;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int j0 = wv; j0 < it.n; j0 += 4 * CB) {
-    T v[CB][2];
-#pragma unroll
-    for (int c = 0; c < CB; ++c)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        v[c][h] = A[(int64_t)min(j0 + 4 * c, it.n - 1) * it.lda + min(lane + 64 * h, it.m - 1)];
-#pragma unroll
-    for (int c = 0; c < CB; ++c)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        if (j0 + 4 * c < it.n && lane + 64 * h < it.m) C[(int64_t)(j0 + 4 * c) * it.ldc + lane + 64 * h] = v[c][h];
   }
 }
 
@@ -251,7 +181,7 @@ __global__ __launch_bounds__(256) void k_copy_tiles(const GemmItem* __restrict__
 // significant bits; TERMS = 1 keeps hi*hi.
 //
 // The BF16 copies are written once per panel, by the kernels that finish it (the diagonal
-// block's by k_potrf_blk, the rows below by the in-place k_gemm<float, true>), in a k-chunked
+// block's by k_potrf_blk, the rows below by k_trsm<float, true>), in a k-chunked
 // layout: entry (i, j) at bpos + ((j / 32) ld + i) 32 + j % 32, zero past the front's width up to
 // a multiple of 32, so a 128-row x 32-column stage of an operand is one contiguous 8 KB block
 // per copy and a product's last stage needs no bounds. The product kernel moves it into LDS with the
@@ -390,7 +320,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
         }
     return;
   }
-  float* C = (it.csrc == S_L ? L : (it.csrc == S_U ? U : Part)) + it.c;
+  float* C = (it.csrc == S_L ? L : U) + it.c;
   // by row blocks, G_SUB's 16 old values of a block loaded first (as in k_gemm)
   const auto rc = raw_rsrc(C);
   const uint32_t ldcb = (uint32_t)it.ldc * sizeof(float);
@@ -414,7 +344,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
         const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<float>::row(lane, v);
         if (i < it.m && j < it.n && i - j + it.diag >= 0) {
           const float x = acc[bi][bj][v] * unscale;
-          C[(int64_t)j * it.ldc + i] = it.mode == G_SUB ? old[bj][v] - x : (it.mode == G_NEG ? -x : x);
+          C[(int64_t)j * it.ldc + i] = it.mode == G_SUB ? old[bj][v] - x : -x;
         }
       }
   }

@@ -257,4 +257,98 @@ __device__ __forceinline__ void substitute_block(typename Mma<M>::acc_t (&x)[NBK
   x[k] = y;
 }
 
+// The rows below a panel's diagonal block, X L11^T = B in place (item: f, a = c0, b = first row):
+// each wave takes sixteen rows through the panel's blocks of sixteen columns in its registers, as
+// substitute_block does, with the factored block's operands read from L and the inverse's diagonal
+// blocks from Inv (both in L2: every wave of the launch reads the same 72 KB) one block row ahead
+// of their use. No LDS, no barrier, and a launch has as many waves as rows / 16, so that the few
+// rows of a small level still spread over the chip: the product with the whole inverse on 128-row
+// tiles gave a level of 2 000 rows 16 workgroups, and the FP64 factor four launches (copy,
+// product, residual, correction) of three times this one's products.
+// SPLIT (mixed form): the rows' scaled BF16 copies too (see k_gemm_b16): a lane's four values of a
+// block are consecutive columns of one row, one 8-byte store a copy; columns from the panel's
+// width up to the next multiple of 32 are zeros (their operands read 0).
+constexpr int TRSM_WAVES = 4;  // waves of a workgroup in launches of many rows (else 1)
+template <typename T, bool SPLIT>
+__global__ __launch_bounds__(64 * TRSM_WAVES) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_trsm(const Item* __restrict__ items,
+                                                          const FrontDev* __restrict__ fronts, T* L,
+                                                          const T* __restrict__ Inv, __bf16* __restrict__ Lh,
+                                                          __bf16* __restrict__ Ll, const int32_t* __restrict__ fexp) {
+  typedef typename Mma<T>::acc_t acc_t;
+  constexpr bool REFINE = sizeof(T) == 8;
+  constexpr int NBK = NB / DB;
+  constexpr uint32_t OUT = 0x80000000u;
+  const Item it = items[blockIdx.x];
+  const FrontDev F = fronts[it.f];
+  const int lane = threadIdx.x & 63, r = lane & 15;
+  const int c0 = it.a, pw = min(NB, F.w - c0), i = it.b + 16 * (int)(threadIdx.x >> 6) + r;
+  const int q0 = Mma<T>::row(lane, 0), dq = Mma<T>::row(lane, 1) - q0;  // a lane's columns of a block: q0 + dq v
+  const bool in = i < F.m;
+  const auto rs = raw_rsrc(L + F.lpos + (int64_t)c0 * F.ld);
+  const auto ri = raw_rsrc(Inv + F.inv0 + (int64_t)(c0 / NB) * NB * NB);
+  const uint32_t ldb = (uint32_t)F.ld * sizeof(T), pwb = (uint32_t)pw * sizeof(T);
+  const uint32_t li = (uint32_t)i * sizeof(T) + q0 * ldb;
+  acc_t x[NBK];
+#pragma unroll
+  for (int k = 0; k < NBK; ++k)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      x[k][v] = buf_load<T>(rs, in && 16 * k + q0 + dq * v < pw ? li : OUT, (16 * k + dq * v) * ldb);
+  // block row k's operands: L_kj (j < k), L_kk^-1 and, to refine, L_kk
+  auto fetch = [&](int k, T (&lo)[NBK][4], T (&xo)[4], T (&dd)[4]) {
+    const bool rin = 16 * k + r < pw;
+    const uint32_t lr = (uint32_t)(c0 + 16 * k + r) * sizeof(T) + q0 * ldb;
+    const uint32_t lx = (uint32_t)(16 * k + r) * sizeof(T) + (16 * k + q0) * pwb;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const bool cin = rin && q0 + dq * s <= r;  // the lower triangle of the diagonal blocks
+      xo[s] = buf_load<T>(ri, cin ? lx : OUT, dq * s * pwb);
+      if (REFINE) dd[s] = buf_load<T>(rs, cin ? lr : OUT, (16 * k + dq * s) * ldb);
+    }
+#pragma unroll
+    for (int j = 0; j < NBK; ++j)
+      if (j < k)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) lo[j][s] = buf_load<T>(rs, rin ? lr : OUT, (16 * j + dq * s) * ldb);
+  };
+  T lo[2][NBK][4], xo[2][4], dd[2][4];
+  fetch(0, lo[0], xo[0], dd[0]);
+#pragma unroll
+  for (int k = 0; k < NBK; ++k) {
+    const int cur = k & 1;
+    if (k + 1 < NBK) fetch(k + 1, lo[cur ^ 1], xo[cur ^ 1], dd[cur ^ 1]);
+    __builtin_amdgcn_sched_barrier(0);  // the next row's loads are issued before this one's products
+    substitute_block<T, REFINE>(
+        x, k, [&](int j, int s) { return lo[cur][j][s]; }, [&](int s) { return xo[cur][s]; },
+        [&](int s) { return dd[cur][s]; });
+  }
+#pragma unroll
+  for (int k = 0; k < NBK; ++k)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      buf_store<T>(rs, (T)x[k][v], in && 16 * k + q0 + dq * v < pw ? li : OUT, (16 * k + dq * v) * ldb);
+  if constexpr (SPLIT) {
+    static_assert(sizeof(T) == 4, "copies of an FP32 result");
+    const float sc = ldexpf(1.0f, -fexp[it.f]);
+    const int ncp = (pw + 31) / 32 * 32;  // c0 is a multiple of 32
+#pragma unroll
+    for (int k = 0; k < NBK; ++k) {
+      const int j = 16 * k + q0;
+      if (in && j < ncp) {
+        __bf16 h[4], l[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float y = (float)x[k][v] * sc;
+          h[v] = (__bf16)y;
+          l[v] = (__bf16)(y - (float)h[v]);
+        }
+        const int col = c0 + j;
+        const int64_t o = F.bpos + ((int64_t)(col / 32) * F.ld + i) * 32 + col % 32;
+        *(uint2*)(Lh + o) = *(const uint2*)h;
+        *(uint2*)(Ll + o) = *(const uint2*)l;
+      }
+    }
+  }
+}
+
 }  // namespace fc

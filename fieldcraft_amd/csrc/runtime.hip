@@ -160,8 +160,8 @@ struct Schedule {
 
 // The launches of the numeric phase and of the solves, built once per analysis.
 struct Program {
-  std::vector<fc::Item> items;         // extend-add and diagonal-block items
-  std::vector<fc::GemmItem> gitems;    // GEMM tiles (UPDATE, TRSM, SYRK launches)
+  std::vector<fc::Item> items;         // extend-add, small-front, diagonal-block and TRSM items
+  std::vector<fc::GemmItem> gitems;    // GEMM tiles (UPDATE, SYRK launches)
   std::vector<fc::ReduceItem> ritems;  // split-K reductions
   std::vector<fc::Launch> launches;
   std::vector<fc::EaRange> earanges;   // extend-add items' child column runs (item.c, item.d)
@@ -170,7 +170,6 @@ struct Program {
   i64 b_size = 0;                      // entries of each BF16 copy
   i64 inv_size = 0;                    // entries of the Inv buffer (kept with the factor)
   i64 part_size = 0;                   // entries of the split-K workspace
-  i64 w_size = 0;                      // entries of the FP64 TRSM workspace
   std::vector<fc::Item> sitems;       // solve work items
   std::vector<fc::Launch> sfwd, sbwd; // forward launches (leaves first), backward (root first)
   std::vector<fc::Launch> sfwd1, sbwd1;  // the same for one right-hand side: each level's block
@@ -182,9 +181,9 @@ struct Program {
   Schedule sched;                     // the schedule the launches were built with
 };
 
-// TRSM launches (Launch.pad): the in-place product run by the FP32 and mixed factors, and the
-// FP64 factor's saved-copy, product, residual and correction steps
-enum TrsmVariant : int32_t { TRSM_IN_PLACE = 0, TRSM_COPY = 1, TRSM_PRODUCT = 2, TRSM_RESIDUAL = 3, TRSM_FIX = 4 };
+// Waves of a TRSM launch from which its workgroups take TRSM_WAVES each: four a SIMD (1 024 SIMDs)
+// keep the chip as busy either way, and a quarter of the items is read.
+constexpr i64 TRSM_WIDE = 4096;
 
 // Side-stream panel updates (Launch.pad of their UPDATE and REDUCE launches): one variant for the
 // FP64 factor, one for the FP32 and mixed ones; each factor runs its own.
@@ -229,7 +228,7 @@ struct Tile {
 constexpr i64 SPLIT_TARGET = 1024;
 constexpr i64 SPLIT_MIN_K = 512;
 
-// One GEMM launch of `tiles` (kind: UPDATE, TRSM or SYRK), split along k when the tiles are
+// One GEMM launch of `tiles` (kind: UPDATE or SYRK), split along k when the tiles are
 // too few, followed by the launch that reduces the pieces.
 void add_gemm(Program& p, const std::vector<Tile>& tiles, int kind, i64 level, i64 split_target = SPLIT_TARGET) {
   if (tiles.empty()) return;
@@ -429,7 +428,7 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
             g.k = (int32_t)(k1 - k0);
             g.mode = fc::G_SUB;
             g.diag = (int32_t)(r - b0);
-            g.asrc = g.bsrc = g.csrc = fc::S_L;
+            g.csrc = fc::S_L;
             g.front = (int32_t)f;
             tiles.push_back(Tile{g, 2.0 * (double)(k1 - k0) * lower_pairs(r, r + m, b0, b1)});
           }
@@ -449,76 +448,23 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
         flops += (double)pw * (pw + 1) * (2 * pw + 1) / 6.0;  // sum_{t <= pw} t^2
       }
       add(fc::K_POTRF, l, i0);
-      // the rows below the diagonal block: X = B Linv^T, in place
-      tiles.clear();
+      // the rows below the diagonal block, sixteen a wave: one wave a workgroup, or TRSM_WAVES of
+      // them (Launch.pad) where single waves would be far more workgroups than the GPU holds at once
+      i64 waves = 0;
+      for (i64 t = 0; t < nl; ++t)
+        if (s.f_w[fl[t]] > c0) waves += (s.f_m[fl[t]] - std::min(c0 + fc::NB, s.f_w[fl[t]]) + 15) / 16;
+      const i64 wpg = waves >= TRSM_WIDE ? fc::TRSM_WAVES : 1;
+      i0 = (i64)p.items.size();
       for (i64 t = 0; t < nl; ++t) {
         const i64 f = fl[t];
         if (s.f_w[f] <= c0) continue;
-        const i64 c1 = std::min(c0 + fc::NB, s.f_w[f]);
-        const i64 pw = c1 - c0;
-        for (i64 r = c1; r < s.f_m[f]; r += fc::GB) {
-          const i64 m = std::min<i64>(fc::GB, s.f_m[f] - r);
-          fc::GemmItem g{};
-          g.a = s.f_lpos[f] + c0 * s.f_ld[f] + r;
-          g.b = p.f_inv0[f] + (c0 / fc::NB) * (i64)fc::NB * fc::NB;
-          g.c = g.a;
-          g.lda = g.ldc = (int32_t)s.f_ld[f];
-          g.ldb = (int32_t)pw;
-          g.m = (int32_t)m;
-          g.n = g.k = (int32_t)pw;
-          g.mode = fc::G_SET;
-          g.diag = fc::GB;
-          g.asrc = g.csrc = fc::S_L;
-          g.bsrc = fc::S_INV;
-          g.front = (int32_t)f;
-          tiles.push_back(Tile{g, (double)m * (double)pw * (double)pw});
-        }
+        const i64 c1 = std::min(c0 + fc::NB, s.f_w[f]), pw = c1 - c0;
+        for (i64 r = c1; r < s.f_m[f]; r += 16 * wpg)
+          p.items.push_back(Item{(int32_t)f, (int32_t)c0, (int32_t)r, 0, 0, 0, 0, 0});
+        flops += (double)(s.f_m[f] - c1) * (double)pw * (double)pw;
       }
-      add_gemm(p, tiles, fc::K_TRSM, l);  // in place (FP32 and mixed factors)
-      // The FP64 factor refines the product once, which makes it as accurate as substitution
-      // (a product with an explicit inverse alone is not backward stable): B is saved in the
-      // workspace W (one GB x GB slot per tile), X = W Linv^T, W -= X L11^T, X += W Linv^T.
-      if (!tiles.empty()) {
-        std::vector<Tile> copy, prod, res, fix;
-        for (size_t q = 0; q < tiles.size(); ++q) {
-          const fc::GemmItem& t = tiles[q].g;
-          const i64 f = t.front, w0 = (i64)q * fc::GB * fc::GB;
-          fc::GemmItem g = t;  // W <- B
-          g.c = w0;
-          g.ldc = fc::GB;
-          g.csrc = fc::S_W;
-          copy.push_back(Tile{g, 0.0});
-          g = t;  // X = W Linv^T
-          g.a = w0;
-          g.lda = fc::GB;
-          g.asrc = fc::S_W;
-          prod.push_back(Tile{g, tiles[q].flops});
-          g = t;  // W -= X L11^T
-          g.a = t.c;
-          g.b = s.f_lpos[f] + (i64)((t.c - s.f_lpos[f]) / s.f_ld[f]) * s.f_ld[f] + (t.c - s.f_lpos[f]) / s.f_ld[f];
-          g.ldb = (int32_t)s.f_ld[f];
-          g.bsrc = fc::S_L;
-          g.c = w0;
-          g.ldc = fc::GB;
-          g.csrc = fc::S_W;
-          g.mode = fc::G_SUB;
-          res.push_back(Tile{g, 0.0});
-          g = t;  // X += W Linv^T
-          g.a = w0;
-          g.lda = fc::GB;
-          g.asrc = fc::S_W;
-          g.mode = fc::G_ADD;
-          fix.push_back(Tile{g, 0.0});
-        }
-        p.w_size = std::max<i64>(p.w_size, (i64)tiles.size() * fc::GB * fc::GB);
-        const double before = p.work[fc::K_TRSM][0];
-        int variant = TRSM_COPY;
-        for (auto* list : {&copy, &prod, &res, &fix}) {
-          add_gemm(p, *list, fc::K_TRSM, l);
-          p.launches.back().pad = variant++;
-        }
-        p.work[fc::K_TRSM][0] = before;  // the algorithmic flops are the in-place product's
-      }
+      add(fc::K_TRSM, l, i0);
+      if ((i64)p.items.size() > i0) p.launches.back().pad = (int32_t)wpg;
     };
     auto sync = [&](int kind, int stream, int slot) {
       Launch q{kind, (int32_t)l, 0, 0, 0, 0.0, 0.0};
@@ -587,7 +533,6 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
           g.k = (int32_t)w;
           g.mode = fc::G_NEG;
           g.diag = (int32_t)(a - b);
-          g.asrc = g.bsrc = fc::S_L;
           g.csrc = fc::S_U;
           g.front = (int32_t)f;
           tiles.push_back(Tile{g, 2.0 * (double)w * lower_pairs(a, a + m, b, b + nn)});
@@ -907,7 +852,6 @@ struct fc_factor {
   unsigned long long* fail = nullptr;
   Buffer U;                // update-matrix arena (kept between factorizations)
   Buffer inv, part;        // diagonal-block inverses, split-K pieces
-  Buffer trsm_w;           // FP64: the rows below a panel, saved for the TRSM's refinement step
   Buffer fexp;             // mixed form: per front, the exponent of its power-of-two scale
   Buffer lb;               // mixed form: BF16 copies (hi, then lo) of the finished panels
   hipGraph_t graph = nullptr;          // opts.use_graph bit 0: the captured factorization
@@ -936,7 +880,6 @@ struct fc_factor {
     U.release();
     inv.release();
     part.release();
-    trsm_w.release();
     fexp.release();
     lb.release();
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
@@ -1086,7 +1029,6 @@ void enqueue_factor(fc_factor* F, const double* dval, i64 nnz, hipStream_t st, b
   const auto& pr = *F->prog;
   T* Inv = (T*)F->inv.get((size_t)std::max<i64>(pr.inv_size, 1) * sizeof(T));
   T* Part = (T*)F->part.get((size_t)std::max<i64>(pr.part_size, 1) * sizeof(T));
-  T* W = F->precision == FC_FP64 ? (T*)F->trsm_w.get((size_t)std::max<i64>(pr.w_size, 1) * sizeof(T)) : nullptr;
   fc::k_fill<T><<<blocks_for(s.l_size), 256, 0, st>>>(L, s.l_size, T(0));
   fc::k_scatter_a<T><<<blocks_for(nnz), 256, 0, st>>>(dval, P.a_pos, nnz, L);
   fc::k_gather_diag<<<blocks_for(s.n), 256, 0, st>>>(dval, P.diag_src, s.n, F->diag);
@@ -1116,7 +1058,6 @@ void enqueue_factor(fc_factor* F, const double* dval, i64 nnz, hipStream_t st, b
       else HIP_CHECK(hipStreamWaitEvent(on, F->sync_ev[l.slot], 0));
       continue;
     }
-    if (l.kind == fc::K_TRSM && (l.pad == TRSM_IN_PLACE) == (F->precision == FC_FP64)) continue;
     if ((l.kind == fc::K_UPDATE || l.kind == fc::K_REDUCE) && l.pad != SIDE_ANY &&
         (l.pad == SIDE_FP64) != (F->precision == FC_FP64))
       continue;  // the other precision's variant of a side-stream update
@@ -1145,20 +1086,17 @@ void enqueue_factor(fc_factor* F, const double* dval, i64 nnz, hipStream_t st, b
             break;
           }
         }
-        fc::k_gemm<T><<<g, b, 0, ls>>>(P.gitems + l.item0, L, U, Inv, Part, W, P.fronts, nullptr, nullptr, nullptr);
+        fc::k_gemm<T><<<g, b, 0, ls>>>(P.gitems + l.item0, L, U, Part);
         break;
       case fc::K_TRSM:
-        if (l.pad == TRSM_COPY) {
-          fc::k_copy_tiles<T><<<g, b, 0, ls>>>(P.gitems + l.item0, L, W);
-        } else {
-          if constexpr (std::is_same<T, float>::value) {
-            if (mixed) {  // the in-place product also writes the rows' BF16 copies
-              fc::k_gemm<T, true><<<g, b, 0, ls>>>(P.gitems + l.item0, L, U, Inv, Part, W, P.fronts, Lh, Ll, fexp);
-              break;
-            }
+        b = dim3(64 * l.pad);
+        if constexpr (std::is_same<T, float>::value) {
+          if (mixed) {  // the rows' BF16 copies too
+            fc::k_trsm<T, true><<<g, b, 0, ls>>>(it, P.fronts, L, Inv, Lh, Ll, fexp);
+            break;
           }
-          fc::k_gemm<T><<<g, b, 0, ls>>>(P.gitems + l.item0, L, U, Inv, Part, W, P.fronts, nullptr, nullptr, nullptr);
         }
+        fc::k_trsm<T, false><<<g, b, 0, ls>>>(it, P.fronts, L, Inv, nullptr, nullptr, nullptr);
         break;
       case fc::K_REDUCE:
         fc::k_reduce_parts<T><<<dim3(l.count * fc::RSPLIT), b, 0, ls>>>(P.ritems + l.item0, L, U, Part);
@@ -1201,7 +1139,6 @@ void run_factor(fc_factor* F, const double* dval, i64 nnz, hipStream_t st) {
       (void)F->U.get((size_t)std::max<i64>(s.u_size, 1) * sizeof(T));
       (void)F->inv.get((size_t)std::max<i64>(pr.inv_size, 1) * sizeof(T));
       (void)F->part.get((size_t)std::max<i64>(pr.part_size, 1) * sizeof(T));
-      if (F->precision == FC_FP64) (void)F->trsm_w.get((size_t)std::max<i64>(pr.w_size, 1) * sizeof(T));
       if (F->precision == FC_MIXED) {
         (void)F->lb.get(2 * (size_t)std::max<i64>(pr.b_size, 1) * sizeof(__bf16));
         (void)F->fexp.get((size_t)std::max<i64>(s.nf, 1) * sizeof(int32_t));
