@@ -79,6 +79,7 @@ struct Launch {
   double entries; // algorithmic entries moved (extend-add: child entries added)
   int32_t stream = 0;  // 0: the caller's stream, 1: the factor's side stream (lookahead)
   int32_t slot = 0;    // event slot of a record / wait step
+  int32_t tile = 0;    // GEMM launches: the output tile's edge
 };
 
 constexpr int KINDS = 8;

@@ -6,8 +6,9 @@
 // (the rows below a panel's diagonal block are panel_kernels.hpp's). A launch with few output tiles is split along k: each piece writes its partial tile (G_PART) and
 // k_reduce_parts adds the pieces in a fixed order, so results do not depend on scheduling.
 //
-// Tile: 128 x 128 per workgroup of 4 waves, each wave a 64 x 64 quarter as 4 x 4 blocks of the
-// 16x16x4 MFMA; k staged 16 at a time in LDS, the next stage prefetched into registers while
+// Tile: TB x TB per workgroup of 4 waves (128, or 64 in launches of few tiles: GB_FEW), each wave a
+// quarter as blocks of the 16x16x4 MFMA; k staged in LDS (16 at a time, 32 for the smaller tile),
+// the next stage prefetched into registers while
 // the current one is multiplied (one barrier a stage). The MFMA's first operand is taken from
 // the j side so that a lane's output column index runs along C's rows: 16 lanes store 16
 // consecutive rows of a column (coalesced, C is column-major).
@@ -21,6 +22,7 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int GB = 128;  // tile edge
+constexpr int GB2 = 64;  // tile edge of launches with few tiles
 constexpr int GK = 16;   // k per LDS stage
 constexpr int NB = 128;  // panel width of the factorization (columns of a diagonal block)
 
@@ -40,10 +42,10 @@ static_assert(sizeof(GemmItem) == 64, "GemmItem layout");
 
 struct ReduceItem {
   int64_t c;              // output offset in csrc
-  int64_t part0;          // first partial tile (GB x GB, column-major) in the split-K workspace
+  int64_t part0;          // first partial tile (tile x tile, column-major) in the split-K workspace
   int32_t ldc, m, n, mode, diag, parts;
   int8_t csrc, pad0, pad1, pad2;
-  int32_t pad3;
+  int32_t tile;           // edge of the partial tiles (TB)
 };
 static_assert(sizeof(ReduceItem) == 48, "ReduceItem layout");
 
@@ -67,23 +69,26 @@ struct Mma<float> {
   static __device__ __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
-template <typename T>
+template <typename T, int TB>
 __global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ items, T* L, T* U, T* Part) {
   constexpr int PAD = 4;
-  __shared__ T As[2][GK][GB + PAD];
-  __shared__ T Bs[2][GK][GB + PAD];
+  constexpr int KS = TB == GB ? GK : 2 * GK;  // k per LDS stage (the same loads a thread either way)
+  constexpr int NQ = TB / 32;                 // 16 x 16 blocks of a wave's quarter, each way
+  constexpr int LK = 256 / TB, LR = KS / LK;  // the loader: a thread one row, every LK-th k
+  __shared__ T As[2][KS][TB + PAD];
+  __shared__ T Bs[2][KS][TB + PAD];
   const GemmItem it = items[blockIdx.x];
   const T* __restrict__ A = L + it.a;
   const T* __restrict__ B = L + it.b;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;
-  const int lrow = tid & (GB - 1), lk = tid >> 7;  // loader: one row, every other k
+  const int wi = (wave >> 1) * (TB / 2), wj = (wave & 1) * (TB / 2);
+  const int lrow = tid & (TB - 1), lk = tid / TB;
   const bool arow = lrow < it.m, brow = lrow < it.n;
-  T ra[GK / 2], rb[GK / 2];
+  T ra[LR], rb[LR];
   auto load = [&](int ks) {
 #pragma unroll
-    for (int r = 0; r < GK / 2; ++r) {
-      const int k = ks + lk + 2 * r;
+    for (int r = 0; r < LR; ++r) {
+      const int k = ks + lk + LK * r;
       const bool kin = k < it.k;
       ra[r] = (arow && kin) ? A[(int64_t)k * it.lda + lrow] : T(0);
       rb[r] = (brow && kin) ? B[(int64_t)k * it.ldb + lrow] : T(0);
@@ -91,35 +96,35 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ it
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int r = 0; r < GK / 2; ++r) {
-      As[buf][lk + 2 * r][lrow] = ra[r];
-      Bs[buf][lk + 2 * r][lrow] = rb[r];
+    for (int r = 0; r < LR; ++r) {
+      As[buf][lk + LK * r][lrow] = ra[r];
+      Bs[buf][lk + LK * r][lrow] = rb[r];
     }
   };
-  typename Mma<T>::acc_t acc[4][4];
+  typename Mma<T>::acc_t acc[NQ][NQ];
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi)
+  for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = typename Mma<T>::acc_t{0, 0, 0, 0};
-  const int stages = (it.k + GK - 1) / GK;
+    for (int bj = 0; bj < NQ; ++bj) acc[bi][bj] = typename Mma<T>::acc_t{0, 0, 0, 0};
+  const int stages = (it.k + KS - 1) / KS;
   load(0);
   store(0);
   __syncthreads();
   for (int s = 0; s < stages; ++s) {
     const int cur = s & 1;
-    if (s + 1 < stages) load((s + 1) * GK);
+    if (s + 1 < stages) load((s + 1) * KS);
 #pragma unroll
-    for (int kk = 0; kk < GK; kk += 4) {
-      T fj[4], fi[4];
+    for (int kk = 0; kk < KS; kk += 4) {
+      T fj[NQ], fi[NQ];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
+      for (int b = 0; b < NQ; ++b) {
         fj[b] = Bs[cur][kk + (lane >> 4)][wj + 16 * b + (lane & 15)];
         fi[b] = As[cur][kk + (lane >> 4)][wi + 16 * b + (lane & 15)];
       }
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
+      for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-        for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = Mma<T>::step(fj[bj], fi[bi], acc[bi][bj]);
+        for (int bj = 0; bj < NQ; ++bj) acc[bi][bj] = Mma<T>::step(fj[bj], fi[bi], acc[bi][bj]);
     }
     if (s + 1 < stages) store(cur ^ 1);
     __syncthreads();
@@ -129,13 +134,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ it
   if (it.mode == G_PART) {
     T* P = Part + it.c;
 #pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
+    for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj)
+      for (int bj = 0; bj < NQ; ++bj)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<T>::row(lane, v);
-          P[(int64_t)j * GB + i] = acc[bi][bj][v];
+          P[(int64_t)j * TB + i] = acc[bi][bj][v];
         }
     return;
   }
@@ -147,11 +152,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ it
   const auto rc = raw_rsrc(C);
   const uint32_t ldcb = (uint32_t)it.ldc * sizeof(T);
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
-    T old[4][4] = {};
+  for (int bi = 0; bi < NQ; ++bi) {
+    T old[NQ][4] = {};
     if (it.mode == G_SUB) {
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj)
+      for (int bj = 0; bj < NQ; ++bj)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<T>::row(lane, v);
@@ -160,7 +165,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const GemmItem* __restrict__ it
         }
     }
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
+    for (int bj = 0; bj < NQ; ++bj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<T>::row(lane, v);
@@ -204,28 +209,60 @@ __device__ __forceinline__ v8bf lds_read16(uint32_t a) {
   return r;
 }
 
-// A product's tile with both operands staged through LDS by direct loads, two stages deep (64
-// KB for three terms: two workgroups share a CU). Stage s lives in buffer s % 2: it is loaded
-// while stage s - 1 is multiplied, then the workgroup waits for its own loads and meets at a
-// barrier (which also frees buffer (s - 1) % 2 for stage s + 1).
+// Fragments of NQ 16-row blocks (1 KB apart) from LDS address a.
+template <int NQ>
+__device__ __forceinline__ void read_rows(v8bf (&f)[NQ], uint32_t a) {
+  f[0] = lds_read16<0>(a);
+  f[1] = lds_read16<1024>(a);
+  if constexpr (NQ == 4) {
+    f[2] = lds_read16<2048>(a);
+    f[3] = lds_read16<3072>(a);
+  }
+}
+
+// Wait until the fragments read above are in their registers (the same statement that names them
+// as changed, so that nothing uses one before).
+__device__ __forceinline__ void frags_wait(v8bf (&a)[2], v8bf (&b)[2]) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]));
+}
+__device__ __forceinline__ void frags_wait(v8bf (&a)[4], v8bf (&b)[4]) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
+}
+__device__ __forceinline__ void frags_wait(v8bf (&a)[2], v8bf (&b)[2], v8bf (&c)[2], v8bf (&d)[2]) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]), "+v"(c[0]), "+v"(c[1]), "+v"(d[0]), "+v"(d[1]));
+}
+__device__ __forceinline__ void frags_wait(v8bf (&a)[4], v8bf (&b)[4], v8bf (&c)[4], v8bf (&d)[4]) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]),
+                 "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]));
+}
+
+// A product's tile (TB x TB) with both operands staged through LDS by direct loads, 64 KB of
+// stages for three terms (two workgroups share a CU): two of a 128 x 128 tile, four of a 64 x 64
+// one, whose launches have few tiles and so wait on each stage's load rather than on the matrix
+// cores.
 //
-// Stage buffer: copy t of A (128 rows x 32 k), then copy t of B. A row's four 16-byte chunks sit
+// Stage buffer: copy t of A (TB rows x 32 k), then copy t of B. A row's four 16-byte chunks sit
 // in the order chunk ^ (row / 2 % 4), the arrangement under which the fragment reads measure
 // free of bank conflicts on gfx950; a wave's direct load fills 1 KB = 16 rows, lane l taking
 // the chunk of LDS slot l.
 // Rows past the tile's m (n) load the last row of the tile (in bounds); their products land in
 // entries that are not stored. The copies are zero past the front's width, so the last stage
 // needs no k bound.
-template <int TERMS>
+template <int TERMS, int TB>
 __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict__ items, const FrontDev* __restrict__ fronts,
                                                      const __bf16* __restrict__ Lh, const __bf16* __restrict__ Ll,
                                                      float* L, float* U, float* Part, const int32_t* __restrict__ fexp) {
   static_assert(TERMS == 1 || TERMS == 3, "one or three BF16 products");
   constexpr int NS = TERMS == 3 ? 2 : 1;       // hi (and lo) copies of each operand
-  constexpr int CE = GB * BK;                  // elements of one copy of one operand per stage
+  constexpr int NQ = TB / 32;                  // 16 x 16 blocks of a wave's quarter, each way
+  constexpr int NBUF = TB == GB ? 2 : 4;       // stage buffers: 64 KB of LDS for three terms
+  constexpr int CE = TB * BK;                  // elements of one copy of one operand per stage
   constexpr int SE = 2 * NS * CE;              // elements of a stage buffer
-  constexpr int PW = 2 * NS * (GB / 16) / 4;   // 1 KB direct loads per wave per stage
-  __shared__ __attribute__((aligned(16))) __bf16 S[2 * SE];
+  constexpr int PW = 2 * NS * (TB / 16) / 4;   // 1 KB direct loads per wave per stage
+  __shared__ __attribute__((aligned(16))) __bf16 S[NBUF * SE];
   const GemmItem it = items[blockIdx.x];
   const FrontDev F = fronts[it.front];
   const int e = fexp[it.front];
@@ -235,13 +272,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
   const int64_t a0 = F.bpos + (oa / F.ld) / BK * chunk + (oa % F.ld) * BK;
   const int64_t b0 = F.bpos + (ob / F.ld) / BK * chunk + (ob % F.ld) * BK;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wi = (wave >> 1) * 64, wj = (wave & 1) * 64;
+  const int wi = (wave >> 1) * (TB / 2), wj = (wave & 1) * (TB / 2);
   const int lrow = lane >> 2, lch = (lane & 3) ^ ((lrow >> 1) & 3);  // the row and chunk slot l holds
   auto issue = [&](int s, int buf) {
 #pragma unroll
     for (int q = 0; q < PW; ++q) {
       const int g = wave + 4 * q;            // which 1 KB block of the stage: operand, copy, rows
-      const int op = g / (NS * GB / 16), t = g / (GB / 16) % NS, rb = g % (GB / 16);
+      const int op = g / (NS * TB / 16), t = g / (TB / 16) % NS, rb = g % (TB / 16);
       const int row = rb * 16 + lrow;
       const int64_t src = (op == 0 ? a0 + (int64_t)min(row, it.m - 1) * BK
                                    : b0 + (int64_t)min(row, it.n - 1) * BK) + s * chunk + lch * 8;
@@ -250,11 +287,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
       __builtin_amdgcn_global_load_lds((const void*)gp, (__attribute__((address_space(3))) void*)lp, 16, 0, 0);
     }
   };
-  v4f acc[4][4];
+  v4f acc[NQ][NQ];
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi)
+  for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = v4f{0, 0, 0, 0};
+    for (int bj = 0; bj < NQ; ++bj) acc[bi][bj] = v4f{0, 0, 0, 0};
   const int stages = (it.k + BK - 1) / BK;
   // a lane's fragment: row lane % 16 of a 16-row block, k chunk lane / 16 (byte offset in a copy)
   const int fr = lane & 15;
@@ -263,46 +300,44 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
   auto mul = [&](int buf) {
     const uint32_t ah = sbase + (uint32_t)(buf * SE + wi * BK) * 2 + foff;
     const uint32_t bh = sbase + (uint32_t)(buf * SE + NS * CE + wj * BK) * 2 + foff;
-    v8bf fi[4], fj[4];
-    fi[0] = lds_read16<0>(ah); fi[1] = lds_read16<1024>(ah); fi[2] = lds_read16<2048>(ah); fi[3] = lds_read16<3072>(ah);
-    fj[0] = lds_read16<0>(bh); fj[1] = lds_read16<1024>(bh); fj[2] = lds_read16<2048>(bh); fj[3] = lds_read16<3072>(bh);
-    if (TERMS == 3) {
-      const uint32_t al = ah + CE * 2, bl = bh + CE * 2;
-      v8bf gi[4], gj[4];
-      gi[0] = lds_read16<0>(al); gi[1] = lds_read16<1024>(al); gi[2] = lds_read16<2048>(al); gi[3] = lds_read16<3072>(al);
-      gj[0] = lds_read16<0>(bl); gj[1] = lds_read16<1024>(bl); gj[2] = lds_read16<2048>(bl); gj[3] = lds_read16<3072>(bl);
-      asm volatile("s_waitcnt lgkmcnt(0)"  // the fragments are in registers
-                   : "+v"(fi[0]), "+v"(fi[1]), "+v"(fi[2]), "+v"(fi[3]), "+v"(fj[0]), "+v"(fj[1]), "+v"(fj[2]),
-                     "+v"(fj[3]), "+v"(gi[0]), "+v"(gi[1]), "+v"(gi[2]), "+v"(gi[3]), "+v"(gj[0]), "+v"(gj[1]),
-                     "+v"(gj[2]), "+v"(gj[3]));
+    v8bf fi[NQ], fj[NQ], gi[NQ], gj[NQ];
+    read_rows<NQ>(fi, ah);
+    read_rows<NQ>(fj, bh);
+    if constexpr (TERMS == 3) {
+      read_rows<NQ>(gi, ah + CE * 2);
+      read_rows<NQ>(gj, bh + CE * 2);
+    }
+    if constexpr (TERMS == 3) frags_wait(fi, fj, gi, gj);
+    else frags_wait(fi, fj);
+    if constexpr (TERMS == 3) {
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
+      for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-        for (int bj = 0; bj < 4; ++bj)
+        for (int bj = 0; bj < NQ; ++bj)
           acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gj[bj], fi[bi], acc[bi][bj], 0, 0, 0);
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
+      for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-        for (int bj = 0; bj < 4; ++bj)
+        for (int bj = 0; bj < NQ; ++bj)
           acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fj[bj], gi[bi], acc[bi][bj], 0, 0, 0);
-    } else {
-      asm volatile("s_waitcnt lgkmcnt(0)"
-                   : "+v"(fi[0]), "+v"(fi[1]), "+v"(fi[2]), "+v"(fi[3]), "+v"(fj[0]), "+v"(fj[1]), "+v"(fj[2]),
-                     "+v"(fj[3]));
     }
 #pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
+    for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj)
+      for (int bj = 0; bj < NQ; ++bj)
         acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fj[bj], fi[bi], acc[bi][bj], 0, 0, 0);
   };
-  if (stages > 0) issue(0, 0);
+  // NBUF - 1 stages in flight: stage s waits for the wave's own loads up to it (those of the NBUF - 2
+  // later stages may be out, PW each; near the end, for all), then meets the others at the
+  // barrier, which also frees buffer (s - 1) % NBUF for stage s + NBUF - 1.
+#pragma unroll
+  for (int s = 0; s < NBUF - 1; ++s)
+    if (s < stages) issue(s, s);
   for (int s = 0; s < stages; ++s) {
-    // this wave's loads of stage s are complete, its LDS reads of stage s - 1 too; after the
-    // barrier every wave's are
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (s + 1 < stages) issue(s + 1, (s + 1) & 1);
-    mul(s & 1);
+    if (s + NBUF - 2 < stages) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NBUF - 2) * PW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s + NBUF - 1 < stages) issue(s + NBUF - 1, (s + NBUF - 1) % NBUF);
+    mul(s % NBUF);
   }
   // acc[bi][bj][v] = C(wi + 16 bi + lane % 16, wj + 16 bj + 4 (lane / 16) + v) / sc^2
   const float unscale = ldexpf(1.0f, 2 * e);
@@ -310,13 +345,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
   if (it.mode == G_PART) {
     float* P = Part + it.c;
 #pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
+    for (int bi = 0; bi < NQ; ++bi)
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj)
+      for (int bj = 0; bj < NQ; ++bj)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<float>::row(lane, v);
-          P[(int64_t)j * GB + i] = acc[bi][bj][v] * unscale;
+          P[(int64_t)j * TB + i] = acc[bi][bj][v] * unscale;
         }
     return;
   }
@@ -325,11 +360,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
   const auto rc = raw_rsrc(C);
   const uint32_t ldcb = (uint32_t)it.ldc * sizeof(float);
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
-    float old[4][4] = {};
+  for (int bi = 0; bi < NQ; ++bi) {
+    float old[NQ][4] = {};
     if (it.mode == G_SUB) {
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj)
+      for (int bj = 0; bj < NQ; ++bj)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<float>::row(lane, v);
@@ -338,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
         }
     }
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
+    for (int bj = 0; bj < NQ; ++bj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int i = wi + 16 * bi + il, j = wj + 16 * bj + Mma<float>::row(lane, v);
@@ -351,7 +386,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_b16(const GemmItem* __restrict_
 }
 
 // Sum of the partial tiles of a split product, in order, applied to C as its mode says. Each
-// tile is shared by RSPLIT workgroups (GB * GB / RSPLIT entries each).
+// tile is shared by RSPLIT workgroups.
 constexpr int RSPLIT = 16;
 
 template <typename T>
@@ -359,10 +394,10 @@ __global__ __launch_bounds__(256) void k_reduce_parts(const ReduceItem* __restri
                                                       const T* __restrict__ Part) {
   const ReduceItem it = items[blockIdx.x / RSPLIT];
   T* C = (it.csrc == S_L ? L : U) + it.c;
-  constexpr int CHUNK = GB * GB / RSPLIT;
-  const int e0 = (blockIdx.x % RSPLIT) * CHUNK;
-  for (int e = e0 + threadIdx.x; e < e0 + CHUNK; e += blockDim.x) {
-    const int i = e % GB, j = e / GB;
+  const int tb = it.tile, tt = tb * tb, chunk = tt / RSPLIT;
+  const int e0 = (blockIdx.x % RSPLIT) * chunk;
+  for (int e = e0 + threadIdx.x; e < e0 + chunk; e += blockDim.x) {
+    const int i = e % tb, j = e / tb;
     if (i >= it.m || j >= it.n || i - j + it.diag < 0) continue;
     T* p = C + (int64_t)j * it.ldc + i;
     const T old = it.mode == G_SUB ? *p : T(0);
@@ -372,11 +407,11 @@ __global__ __launch_bounds__(256) void k_reduce_parts(const ReduceItem* __restri
     for (; q + 8 <= it.parts; q += 8) {
       T v[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) v[t] = Part[it.part0 + (int64_t)(q + t) * GB * GB + e];
+      for (int t = 0; t < 8; ++t) v[t] = Part[it.part0 + (int64_t)(q + t) * tt + e];
 #pragma unroll
       for (int t = 0; t < 8; ++t) s += v[t];
     }
-    for (; q < it.parts; ++q) s += Part[it.part0 + (int64_t)q * GB * GB + e];
+    for (; q < it.parts; ++q) s += Part[it.part0 + (int64_t)q * tt + e];
     *p = it.mode == G_SUB ? old - s : -s;
   }
 }

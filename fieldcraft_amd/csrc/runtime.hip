@@ -223,14 +223,18 @@ struct Tile {
   double flops;
 };
 
-// Output tiles a launch should have to fill the GPU (256 CUs, two workgroups each, and some
-// slack); a launch with fewer is split along k into pieces of at least SPLIT_MIN_K.
-constexpr i64 SPLIT_TARGET = 1024;
+// A launch with fewer output tiles than its split target is split along k into pieces of at least
+// SPLIT_MIN_K.
 constexpr i64 SPLIT_MIN_K = 512;
+// GEMM launches of at most this many 128 x 128 tiles take 64 x 64 ones instead (four times the
+// workgroups, a quarter of the work each): below one tile a CU a launch's time is its tile's own
+// chain of stages, and one FP64 tile 128 deep is 14 us of a CU's matrix cores. Measured, launches of
+// the 40 x 8 x 8 cantilever's FP64 factor 46 -> 17 us; BF16 ones of the 40^3 cube at most 18 us.
+constexpr i64 GB_FEW = 192;
 
 // One GEMM launch of `tiles` (kind: UPDATE or SYRK), split along k when the tiles are
 // too few, followed by the launch that reduces the pieces.
-void add_gemm(Program& p, const std::vector<Tile>& tiles, int kind, i64 level, i64 split_target = SPLIT_TARGET) {
+void add_gemm(Program& p, const std::vector<Tile>& tiles, int kind, i64 level, i64 split_target, i64 tb) {
   if (tiles.empty()) return;
   const i64 nt = (i64)tiles.size();
   const i64 g0 = (i64)p.gitems.size(), r0 = (i64)p.ritems.size();
@@ -260,6 +264,7 @@ void add_gemm(Program& p, const std::vector<Tile>& tiles, int kind, i64 level, i
     r.diag = t.g.diag;
     r.parts = (int32_t)split;
     r.csrc = t.g.csrc;
+    r.tile = (int32_t)tb;
     p.ritems.push_back(r);
     for (i64 q = 0; q < split; ++q) {
       fc::GemmItem g = t.g;
@@ -267,13 +272,14 @@ void add_gemm(Program& p, const std::vector<Tile>& tiles, int kind, i64 level, i
       g.b += q * chunk * (i64)t.g.ldb;
       g.k = (int32_t)std::min<i64>(chunk, t.g.k - q * chunk);
       g.mode = fc::G_PART;
-      g.c = part + q * (i64)fc::GB * fc::GB;
+      g.c = part + q * tb * tb;
       g.csrc = fc::S_PART;
       p.gitems.push_back(g);
     }
-    part += split * (i64)fc::GB * fc::GB;
+    part += split * tb * tb;
   }
   p.launches.push_back(fc::Launch{kind, (int32_t)level, g0, (int32_t)((i64)p.gitems.size() - g0), 0, flops, 0.0});
+  p.launches.back().tile = (int32_t)tb;
   p.work[kind][0] += flops;
   if ((i64)p.ritems.size() > r0)
     p.launches.push_back(fc::Launch{fc::K_REDUCE, (int32_t)level, r0, (int32_t)((i64)p.ritems.size() - r0), 0, 0.0, 0.0});
@@ -412,12 +418,16 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
     // [k0, k1) (all before c0): one tile column per panel, from the panel's diagonal down.
     auto update = [&](i64 c0, i64 c1, i64 k0, i64 k1, i64 split_target) {
       tiles.clear();
+      i64 nt = 0;
+      for (i64 t = 0; t < nl; ++t)
+        for (i64 b0 = c0; b0 < std::min(c1, s.f_w[fl[t]]); b0 += fc::GB) nt += (s.f_m[fl[t]] - b0 + fc::GB - 1) / fc::GB;
+      const i64 tb = nt <= GB_FEW ? fc::GB2 : fc::GB;
       for (i64 t = 0; t < nl; ++t) {
         const i64 f = fl[t];
-        for (i64 b0 = c0; b0 < std::min(c1, s.f_w[f]); b0 += fc::NB) {
-          const i64 b1 = std::min(b0 + fc::NB, s.f_w[f]);
-          for (i64 r = b0; r < s.f_m[f]; r += fc::GB) {
-            const i64 m = std::min<i64>(fc::GB, s.f_m[f] - r);
+        for (i64 b0 = c0; b0 < std::min(c1, s.f_w[f]); b0 += tb) {
+          const i64 b1 = std::min(b0 + tb, s.f_w[f]);
+          for (i64 r = b0; r < s.f_m[f]; r += tb) {
+            const i64 m = std::min<i64>(tb, s.f_m[f] - r);
             fc::GemmItem g{};
             g.a = s.f_lpos[f] + k0 * s.f_ld[f] + r;
             g.b = s.f_lpos[f] + k0 * s.f_ld[f] + b0;
@@ -434,7 +444,7 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
           }
         }
       }
-      add_gemm(p, tiles, fc::K_UPDATE, l, split_target);
+      add_gemm(p, tiles, fc::K_UPDATE, l, split_target, tb);
     };
     // The panel at c0 once its updates are in: diagonal block, rows below, BF16 copies.
     auto chain = [&](i64 c0) {
@@ -516,12 +526,18 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
     }
     // update matrices U = -L21 L21^T
     tiles.clear();
+    i64 nt = 0;
+    for (i64 t = 0; t < nl; ++t) {
+      const i64 q = (s.f_m[fl[t]] - s.f_w[fl[t]] + fc::GB - 1) / fc::GB;
+      nt += q * (q + 1) / 2;
+    }
+    const i64 tb = nt <= GB_FEW ? fc::GB2 : fc::GB;
     for (i64 t = 0; t < nl; ++t) {
       const i64 f = fl[t];
       const i64 w = s.f_w[f], mu = s.f_m[f] - w;
-      for (i64 a = 0; a < mu; a += fc::GB)
-        for (i64 b = 0; b <= a; b += fc::GB) {
-          const i64 m = std::min<i64>(fc::GB, mu - a), nn = std::min<i64>(fc::GB, mu - b);
+      for (i64 a = 0; a < mu; a += tb)
+        for (i64 b = 0; b <= a; b += tb) {
+          const i64 m = std::min<i64>(tb, mu - a), nn = std::min<i64>(tb, mu - b);
           fc::GemmItem g{};
           g.a = s.f_lpos[f] + w + a;
           g.b = s.f_lpos[f] + w + b;
@@ -538,7 +554,7 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
           tiles.push_back(Tile{g, 2.0 * (double)w * lower_pairs(a, a + m, b, b + nn)});
         }
     }
-    add_gemm(p, tiles, fc::K_SYRK, l, sched.split_target);
+    add_gemm(p, tiles, fc::K_SYRK, l, sched.split_target, tb);
     i0 = (i64)p.items.size();
     for (i64 t = 0; t < nall; ++t) {
       const i64 f = fall[t];
@@ -1079,14 +1095,22 @@ void enqueue_factor(fc_factor* F, const double* dval, i64 nnz, hipStream_t st, b
       case fc::K_SYRK:
         if constexpr (std::is_same<T, float>::value) {
           if (mixed) {
-            if (F->opts.bf16_terms == 1)
-              fc::k_gemm_b16<1><<<g, b, 0, ls>>>(P.gitems + l.item0, P.fronts, Lh, Ll, L, U, Part, fexp);
-            else
-              fc::k_gemm_b16<3><<<g, b, 0, ls>>>(P.gitems + l.item0, P.fronts, Lh, Ll, L, U, Part, fexp);
+            auto b16 = [&](auto terms, auto tb) {
+              fc::k_gemm_b16<decltype(terms)::value, decltype(tb)::value>
+                  <<<g, b, 0, ls>>>(P.gitems + l.item0, P.fronts, Lh, Ll, L, U, Part, fexp);
+            };
+            typedef std::integral_constant<int, fc::GB> Large;
+            typedef std::integral_constant<int, fc::GB2> Few;
+            typedef std::integral_constant<int, 1> One;
+            typedef std::integral_constant<int, 3> Three;
+            const bool one = F->opts.bf16_terms == 1;
+            if (l.tile == fc::GB) one ? b16(One{}, Large{}) : b16(Three{}, Large{});
+            else one ? b16(One{}, Few{}) : b16(Three{}, Few{});
             break;
           }
         }
-        fc::k_gemm<T><<<g, b, 0, ls>>>(P.gitems + l.item0, L, U, Part);
+        if (l.tile == fc::GB) fc::k_gemm<T, fc::GB><<<g, b, 0, ls>>>(P.gitems + l.item0, L, U, Part);
+        else fc::k_gemm<T, fc::GB2><<<g, b, 0, ls>>>(P.gitems + l.item0, L, U, Part);
         break;
       case fc::K_TRSM:
         b = dim3(64 * l.pad);
