@@ -84,14 +84,18 @@ struct Launch {
 
 constexpr int KINDS = 8;
 
-// A child's run of update-matrix columns landing in an extend-add item's parent columns:
-// columns [jc0, jc1) of child front `child`.
+// A child's run of update-matrix columns landing in a window of an extend-add item's parent columns:
+// columns [jc0, jc1) of the child's cmu, its update matrix at u and its row map at rel.
 struct EaRange {
-  int32_t child, jc0, jc1, pad;
+  int64_t u, rel;
+  int32_t cmu, jc0, jc1;
+  int32_t win;  // the window's first parent column
 };
+static_assert(sizeof(EaRange) == 32, "EaRange layout");
 
-constexpr int EA_BATCH = 8;   // rows an extend-add thread moves at a time
-constexpr int EA_COLS = 8;     // columns of the parent an extend-add window spans
-constexpr int EA_ENTRIES = 8192;  // child entries an extend-add workgroup takes (whole windows)
+constexpr int EA_BATCH = 4;       // rows a lane moves at a time, of each of its columns
+constexpr int EA_COLS = 8;        // columns of the parent an extend-add window spans (two a wave)
+constexpr int EA_ENTRIES = 8192;  // child entries an extend-add workgroup takes (whole windows) where
+                                  // a launch has many
 
 }  // namespace fc

@@ -69,76 +69,73 @@ __global__ void k_fill(T* __restrict__ p, int64_t len, T v) {
 // matrix entries that land there, child after child (in increasing order), so each entry
 // receives its contributions in a fixed order and no two workgroups write the same entry.
 // Item: f, a, b, and at ranges[c .. c + d) the children's column runs that land in [a, b),
-// window of EA_COLS parent columns after window, children in increasing order within a
+// window of at most EA_COLS parent columns after window, children in increasing order within a
 // window (children with none are not listed; the runs are found when the launches are planned).
-
+//
+// Wave v takes the window's columns win + v and win + v + 4, through every child: a column's entries
+// stay with one wave, whose memory operations are in order, so the children need no barrier. Lanes
+// run along the child's rows, both columns together (one read of the row map for the two), EA_BATCH
+// rows of each in flight. Bound: HBM, 12 bytes a child's FP32 entry (20 FP64) and the row maps; in
+// levels of few columns, the chain of a workgroup's ranges (three memory round trips each). Taken
+// as one flat range of 8 columns by the whole workgroup, with a barrier after each child and
+// selects to find an entry's column, a launch of the cantilever's FP64 factor took 64 us (now 9), of
+// the 28^3 cube's 91 us (57), of the 40^3 cube's mixed one 136 us (100).
 template <typename T>
 __global__ __launch_bounds__(256) void k_extend_add(const Item* __restrict__ items, const EaRange* __restrict__ ranges,
                                                     const FrontDev* __restrict__ fronts,
-                                                    const int32_t* __restrict__ rel, T* __restrict__ L, const T* U,
+                                                    const int32_t* __restrict__ rel, T* L, const T* __restrict__ U,
                                                     T* Uw) {
   // U (children, read) and Uw (this front, written) are disjoint blocks of one arena
   const Item it = items[blockIdx.x];
   const FrontDev P = fronts[it.f];
-  const int pw = P.w;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t pmu = P.m - P.w;
   for (int q = it.c; q < it.c + it.d; ++q) {
     const EaRange rg = ranges[q];
-    const FrontDev C = fronts[rg.child];
-    const int cmu = C.m - C.w;
-    const int32_t* r = rel + C.rel_off;
-    const int jc0 = rg.jc0, jc1 = rg.jc1;  // child columns whose parent column lies in [a, b)
-    const T* cu = U + C.upos;
-    // The child's entries that land in [j0, j1): columns jc0 + t (t < nc <= EA_COLS, rel is
-    // injective), rows jc0 + t .. cmu - 1 of each, taken as one flat range so that small
-    // children still fill the workgroup. Entry e of the range is column t with
-    // off[t] <= e < off[t + 1], row jc0 + t + e - off[t].
-    const int nc = jc1 - jc0;
-    int off[EA_COLS + 1];
-    T* dcol[EA_COLS];
-    off[0] = 0;
+    const int32_t* r = rel + rg.rel;
+    // the child's columns that land on the wave's two: lane l looks at column jc0 + l
+    const int mine = lane < rg.jc1 - rg.jc0 ? r[rg.jc0 + lane] - rg.win - wave : -1;
+    const uint64_t m0 = __ballot(mine == 0), m1 = __ballot(mine == 4);
+    if (!(m0 | m1)) continue;
+    int jc[2];
+    T* d[2];
+    const T* s[2];
 #pragma unroll
-    for (int t = 0; t < EA_COLS; ++t) {
-      const int jc = min(jc0 + min(t, max(nc - 1, 0)), cmu - 1);  // in bounds
-      off[t + 1] = off[t] + (t < nc ? cmu - (jc0 + t) : 0);
-      const int jp = nc > 0 ? r[jc] : 0;
-      dcol[t] = jp < pw ? L + P.lpos + (int64_t)jp * P.ld : Uw + P.upos + (int64_t)(jp - pw) * pmu - pw;
+    for (int h = 0; h < 2; ++h) {
+      const uint64_t m = h ? m1 : m0;
+      const int p = rg.win + wave + 4 * h;
+      jc[h] = m ? rg.jc0 + __ffsll((unsigned long long)m) - 1 : rg.cmu;  // none: no row
+      d[h] = p < P.w ? L + P.lpos + (int64_t)p * P.ld : Uw + P.upos + (int64_t)(p - P.w) * pmu - P.w;
+      s[h] = U + rg.u + (int64_t)min(jc[h], rg.cmu - 1) * rg.cmu;
     }
-    const int total = off[EA_COLS];
-    // EA_BATCH entries a thread at a time: the row map and the child's entries, then the
-    // targets, then the sums (distinct targets within one child). Entries past the range read
-    // its last entry (in bounds) and store nothing.
-    for (int e0 = threadIdx.x; e0 < total; e0 += EA_BATCH * blockDim.x) {
-      int ri[EA_BATCH], tc[EA_BATCH];
-      T sv[EA_BATCH], dv[EA_BATCH];
+    // rows from the first column's on; a lane's rows past the range read its last one (in bounds)
+    // and store nothing
+    for (int i0 = min(jc[0], jc[1]) + lane; i0 < rg.cmu; i0 += 64 * EA_BATCH) {
+      int ri[EA_BATCH];
+      T sv[2][EA_BATCH], dv[2][EA_BATCH];
 #pragma unroll
       for (int k = 0; k < EA_BATCH; ++k) {
-        const int e = min(e0 + k * (int)blockDim.x, total - 1);
-        int t = 0;
+        const int i = min(i0 + 64 * k, rg.cmu - 1);
+        ri[k] = r[i];
 #pragma unroll
-        for (int q2 = 1; q2 < EA_COLS; ++q2) t += e >= off[q2];
-        const int ic = jc0 + t + e - off[t];
-        tc[k] = t;
-        ri[k] = r[ic];
-        sv[k] = cu[(int64_t)(jc0 + t) * cmu + ic];
-      }
-#pragma unroll
-      for (int k = 0; k < EA_BATCH; ++k) {
-        T* d = dcol[0];
-#pragma unroll
-        for (int q2 = 1; q2 < EA_COLS; ++q2) d = tc[k] == q2 ? dcol[q2] : d;
-        dv[k] = d[ri[k]];
+        for (int h = 0; h < 2; ++h) sv[h][k] = i >= jc[h] ? s[h][i] : T(0);
       }
 #pragma unroll
       for (int k = 0; k < EA_BATCH; ++k)
-        if (e0 + k * (int)blockDim.x < total) {
-          T* d = dcol[0];
 #pragma unroll
-          for (int q2 = 1; q2 < EA_COLS; ++q2) d = tc[k] == q2 ? dcol[q2] : d;
-          d[ri[k]] = dv[k] + sv[k];
+        for (int h = 0; h < 2; ++h) {
+          const int i = i0 + 64 * k;
+          dv[h][k] = (i < rg.cmu && i >= jc[h]) ? d[h][ri[k]] : T(0);
+        }
+#pragma unroll
+      for (int k = 0; k < EA_BATCH; ++k)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int i = i0 + 64 * k;
+          if (i < rg.cmu && i >= jc[h]) d[h][ri[k]] = dv[h][k] + sv[h][k];
         }
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the next child's loads stay behind these stores
   }
 }
 

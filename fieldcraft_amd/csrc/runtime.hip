@@ -232,6 +232,9 @@ constexpr i64 SPLIT_MIN_K = 512;
 // the 40 x 8 x 8 cantilever's FP64 factor 46 -> 17 us; BF16 ones of the 40^3 cube at most 18 us.
 constexpr i64 GB_FEW = 192;
 
+// Workgroups an extend-add launch is divided into where its columns allow (four a CU).
+constexpr i64 EA_ITEMS = 1024;
+
 // One GEMM launch of `tiles` (kind: UPDATE or SYRK), split along k when the tiles are
 // too few, followed by the launch that reduces the pieces.
 void add_gemm(Program& p, const std::vector<Tile>& tiles, int kind, i64 level, i64 split_target, i64 tb) {
@@ -331,7 +334,6 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
     const i64 full = s.f_w[f] / fc::NB, last = s.f_w[f] % fc::NB;
     p.inv_size += full * fc::NB * fc::NB + last * last;
   }
-  std::vector<double> colent;  // child entries landing in each parent column
   for (i64 l = 0; l < s.levels; ++l) {
     // the level's fronts (every one takes the extend-add launches), its small fronts
     // (k_small_fronts) and the others (the tiled launches)
@@ -346,18 +348,12 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
         if (s.f_m[s.f_kids[q]] > s.f_w[s.f_kids[q]]) return true;
       return false;
     };
-    auto column_entries = [&](i64 f) {
-      colent.assign(s.f_m[f], 0.0);
-      for (i64 q = s.f_kptr[f]; q < s.f_kptr[f + 1]; ++q) {
-        const i64 c = s.f_kids[q], cmu = s.f_m[c] - s.f_w[c];
-        for (i64 jc = 0; jc < cmu; ++jc) colent[s.rel[s.f_rel_off[c] + jc]] += (double)(cmu - jc);
-      }
-    };
-    // Extend-add items: windows of EA_COLS parent columns, each with the runs of its children's
-    // columns that land there (rel rises, so each child's is one run), children in increasing
-    // order. Consecutive windows of one front share an item until it holds EA_ENTRIES child
-    // entries, so that small fronts still give a workgroup enough to move.
-    i64 ea_r0 = -1, ea_n = 0;
+    // Extend-add items: windows of parent columns (at most EA_COLS), each with the runs of its
+    // children's columns that land there (rel rises, so each child's is one run), children in
+    // increasing order. Consecutive windows of one front share an item until it holds `ea_min`
+    // child entries, so that small fronts still give a workgroup enough to move; a level with
+    // little to move takes single windows, of half the columns (one a wave) below EA_ITEMS windows.
+    i64 ea_r0 = -1, ea_n = 0, ea_min = fc::EA_ENTRIES;
     int32_t ea_f = -1, ea_a = 0, ea_b = 0;
     auto ea_close = [&]() {
       if (ea_r0 >= 0 && (i64)p.earanges.size() > ea_r0)
@@ -366,7 +362,7 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
       ea_n = 0;
     };
     auto ea_window = [&](i64 f, i64 a, i64 b) {
-      if (ea_r0 >= 0 && (ea_f != (int32_t)f || ea_n >= fc::EA_ENTRIES)) ea_close();
+      if (ea_r0 >= 0 && (ea_f != (int32_t)f || ea_n >= ea_min)) ea_close();
       if (ea_r0 < 0) {
         ea_r0 = (i64)p.earanges.size();
         ea_f = (int32_t)f;
@@ -378,24 +374,45 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
         const int32_t* rc = s.rel.data() + s.f_rel_off[c];
         const i64 jc0 = std::lower_bound(rc, rc + cmu, (int32_t)a) - rc;
         const i64 jc1 = std::lower_bound(rc + jc0, rc + cmu, (int32_t)b) - rc;
-        if (jc1 > jc0) p.earanges.push_back(fc::EaRange{(int32_t)c, (int32_t)jc0, (int32_t)jc1, 0});
+        if (jc1 > jc0)
+          p.earanges.push_back(fc::EaRange{s.f_upos[c], s.f_rel_off[c], (int32_t)cmu, (int32_t)jc0, (int32_t)jc1, (int32_t)a});
         for (i64 jc = jc0; jc < jc1; ++jc) ea_n += cmu - jc;
       }
     };
-    // extend-add into the L parts
-    i64 i0 = (i64)p.items.size();
-    for (i64 t = 0; t < nall; ++t) {
-      const i64 f = fall[t];
-      if (!has_kids_below(f)) continue;
-      column_entries(f);
-      for (i64 a = 0; a < s.f_w[f]; a += fc::EA_COLS) {
-        const i64 b = std::min(a + fc::EA_COLS, s.f_w[f]);
-        ea_window(f, a, b);
-        for (i64 j = a; j < b; ++j) entries += colent[j];
+    // one extend-add launch: into the fronts' L parts, or their update matrices
+    auto extend = [&](int kind) {
+      auto range = [&](i64 f) {
+        return kind == fc::K_EXTEND_L ? std::make_pair((i64)0, s.f_w[f]) : std::make_pair(s.f_w[f], s.f_m[f]);
+      };
+      double total = 0;
+      i64 cols = 0;
+      for (i64 t = 0; t < nall; ++t) {
+        const i64 f = fall[t];
+        if (!has_kids_below(f)) continue;
+        const auto [a, b] = range(f);
+        cols += b - a;
+        for (i64 q = s.f_kptr[f]; q < s.f_kptr[f + 1]; ++q) {  // the children's columns that land in [a, b)
+          const i64 c = s.f_kids[q], cmu = s.f_m[c] - s.f_w[c];
+          const int32_t* rc = s.rel.data() + s.f_rel_off[c];
+          const i64 j0 = std::lower_bound(rc, rc + cmu, (int32_t)a) - rc, j1 = std::lower_bound(rc, rc + cmu, (int32_t)b) - rc;
+          total += 0.5 * (double)(j1 - j0) * (double)(2 * cmu - j0 - j1 + 1);
+        }
       }
-    }
-    ea_close();
-    add(fc::K_EXTEND_L, l, i0);
+      ea_min = std::min<i64>(fc::EA_ENTRIES, (i64)(total / EA_ITEMS));
+      const i64 wc = cols < EA_ITEMS * fc::EA_COLS ? fc::EA_COLS / 2 : fc::EA_COLS;
+      const i64 i0 = (i64)p.items.size();
+      for (i64 t = 0; t < nall; ++t) {
+        const i64 f = fall[t];
+        if (!has_kids_below(f)) continue;
+        const auto [lo, hi] = range(f);
+        for (i64 a = lo; a < hi; a += wc) ea_window(f, a, std::min(a + wc, hi));
+      }
+      ea_close();
+      entries = total;
+      add(kind, l, i0);
+    };
+    extend(fc::K_EXTEND_L);
+    i64 i0 = 0;
     // the small fronts' diagonal blocks, rows below and update matrices, one item (workgroup)
     // each, costliest first (the first workgroups to start take them)
     auto small_cost = [&](i64 f) {
@@ -555,19 +572,7 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
         }
     }
     add_gemm(p, tiles, fc::K_SYRK, l, sched.split_target, tb);
-    i0 = (i64)p.items.size();
-    for (i64 t = 0; t < nall; ++t) {
-      const i64 f = fall[t];
-      if (!has_kids_below(f)) continue;
-      column_entries(f);
-      for (i64 a = s.f_w[f]; a < s.f_m[f]; a += fc::EA_COLS) {
-        const i64 b = std::min(a + fc::EA_COLS, s.f_m[f]);
-        ea_window(f, a, b);
-        for (i64 j = a; j < b; ++j) entries += colent[j];
-      }
-    }
-    ea_close();
-    add(fc::K_EXTEND_U, l, i0);
+    extend(fc::K_EXTEND_U);
   }
   // solves: per level, forward leaves first, backward root first
   auto sadd = [&](std::vector<Launch>& list, int kind, i64 level, i64 item0) {
