@@ -172,8 +172,6 @@ struct Program {
   i64 part_size = 0;                   // entries of the split-K workspace
   std::vector<fc::Item> sitems;       // solve work items
   std::vector<fc::Launch> sfwd, sbwd; // forward launches (leaves first), backward (root first)
-  std::vector<fc::Launch> sfwd1, sbwd1;  // the same for one right-hand side: each level's block
-                                         // chain in one launch (k_fwd_front / k_bwd_front)
 
   std::vector<i64> uoff;              // per front: start of its solve contribution
   i64 u_solve = 0;                    // total contribution length (one right-hand side)
@@ -197,18 +195,20 @@ constexpr int32_t L_WAIT = 101;
 constexpr int SYNC_SLOTS = 4;
 
 // kinds of solve launches
-enum SolveKind : int32_t {
-  S_GATHER = 0,
-  S_FWD_STEP = 1,
-  S_BWD_GATHER = 2,
-  S_BWD_BELOW = 3,
-  S_BWD_FIRST = 4,
-  S_BWD_STEP = 5,
-  S_FWD_FRONT = 6,
-  S_BWD_FRONT = 7
-};
+enum SolveKind : int32_t { S_FWD = 0, S_FWD_ONE = 1, S_BELOW = 2, S_BWD = 3, S_BWD_ONE = 4 };
 static_assert(fc::SNB == fc::NB, "solve blocks are the factorization's panels");
-static_assert(fc::BCOLS == fc::SNB, "a backward column tile is one block");
+
+// In a level with wider fronts, one-block fronts of up to this many workgroups in all take the wide
+// fronts' launch (each launch of a level is another dependent step); more take one of their own,
+// whose kernel keeps more workgroups on a CU.
+constexpr i64 ONE_FEW = 256;
+// One-block fronts' forward workgroups take ONE_ROWS rows, or a quarter of that in launches of fewer
+// than ONE_MANY workgroups (a workgroup takes its rows 64 at a time, several memory round trips
+// each; every one forms the block's y again).
+constexpr i64 ONE_MANY = 2048;
+// Launches of the products with the rows below take 16 columns a workgroup instead of 32 where there are
+// fewer than this many.
+constexpr i64 SOLVE_FEW = 512;
 
 // lower pairs (i >= j) of rows [r0, r1) x columns [c0, c1)
 double lower_pairs(i64 r0, i64 r1, i64 c0, i64 c1) {
@@ -575,130 +575,84 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
     extend(fc::K_EXTEND_U);
   }
   // solves: per level, forward leaves first, backward root first
-  auto sadd = [&](std::vector<Launch>& list, int kind, i64 level, i64 item0) {
+  if (s.f_rptr[s.nf] >= (i64)UINT32_MAX || s.s_size >= (i64)UINT32_MAX)
+    throw fc::Failure{fc::TOO_LARGE, -1, s.s_size, (i64)UINT32_MAX - 1, "a solve's rows pass 2^32"};
+  auto sadd = [&](std::vector<Launch>& list, int kind, i64 level, i64 item0, int32_t pad = 0) {
     const i64 count = (i64)p.sitems.size() - item0;
-    if (count > 0) list.push_back(Launch{kind, (int32_t)level, item0, (int32_t)count, 0, 0.0, 0.0});
+    if (count > 0) list.push_back(Launch{kind, (int32_t)level, item0, (int32_t)count, pad, 0.0, 0.0});
+  };
+  auto sitem = [&](i64 f, i64 a, i64 b) {
+    p.sitems.push_back(Item{(int32_t)f, (int32_t)a, (int32_t)b, 0, 0, 0, 0, 0});
+  };
+  auto blocks = [&](i64 f) { return (s.f_w[f] + fc::SNB - 1) / fc::SNB; };
+  // a level's fronts: those of the wide fronts' launches, and the one-block fronts of their own
+  std::vector<i64> wide, one;
+  auto sort_level = [&](i64 l) {
+    wide.clear();
+    one.clear();
+    i64 tiles = 0;
+    for (i64 q = s.lvl_ptr[l]; q < s.lvl_ptr[l + 1]; ++q) {
+      const i64 f = s.lvl_fronts[q];
+      (blocks(f) > 1 ? wide : one).push_back(f);
+      if (blocks(f) <= 1) tiles += (s.f_m[f] + fc::SNB - 1) / fc::SNB;
+    }
+    if (!wide.empty() && tiles <= ONE_FEW) {
+      wide.insert(wide.end(), one.begin(), one.end());
+      one.clear();
+    }
   };
   for (i64 l = 0; l < s.levels; ++l) {
-    const i64* fl = &s.lvl_fronts[s.lvl_ptr[l]];
-    const i64 nl = s.lvl_ptr[l + 1] - s.lvl_ptr[l];
-    i64 wmax = 0;
-    for (i64 t = 0; t < nl; ++t) wmax = std::max(wmax, s.f_w[fl[t]]);
+    sort_level(l);
     i64 i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t) p.sitems.push_back(Item{(int32_t)fl[t], 0, 0, 0, 0, 0, 0, 0});
-    sadd(p.sfwd, S_GATHER, l, i0);
-    for (i64 c0 = 0; c0 < wmax; c0 += fc::SNB) {
-      i0 = (i64)p.sitems.size();
-      for (i64 t = 0; t < nl; ++t) {
-        const i64 f = fl[t];
-        if (s.f_w[f] <= c0) continue;
-        const i64 c1 = std::min(c0 + fc::SNB, s.f_w[f]);
-        // the first row tile also forms the next block's solution
-        for (i64 r = c1; r < s.f_m[f]; r += fc::SROWS_M)
-          p.sitems.push_back(Item{(int32_t)f, (int32_t)c0, (int32_t)r, (r == c1 && c1 < s.f_w[f]) ? 1 : 0, 0, 0, 0, 0});
-      }
-      sadd(p.sfwd, S_FWD_STEP, l, i0);
+    i64 count = 0, rows = fc::ONE_ROWS;
+    for (const i64 f : one) count += (s.f_m[f] + rows - 1) / rows;
+    if (count < ONE_MANY) rows /= 4;
+    for (const i64 f : one) {
+      // the first workgroup takes the block's rows' share too
+      for (i64 a = 0; a < s.f_m[f]; a += rows)
+        if (a == 0 || a + rows > s.f_w[f]) sitem(f, a, std::min(a + rows, s.f_m[f]));
     }
-  }
-  for (i64 l = s.levels - 1; l >= 0; --l) {
-    const i64* fl = &s.lvl_fronts[s.lvl_ptr[l]];
-    const i64 nl = s.lvl_ptr[l + 1] - s.lvl_ptr[l];
-    i64 wmax = 0;
-    i64 i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t)
-      if (s.f_m[fl[t]] > s.f_w[fl[t]]) p.sitems.push_back(Item{(int32_t)fl[t], 0, 0, 0, 0, 0, 0, 0});
-    sadd(p.sbwd, S_BWD_GATHER, l, i0);
-    i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t) {
-      const i64 f = fl[t];
-      wmax = std::max(wmax, s.f_w[f]);
-      if (s.f_m[f] == s.f_w[f]) continue;
-      for (i64 j = 0; j < s.f_w[f]; j += fc::SCOLS) p.sitems.push_back(Item{(int32_t)f, (int32_t)j, 0, 0, 0, 0, 0, 0});
-    }
-    sadd(p.sbwd, S_BWD_BELOW, l, i0);
-    i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t) p.sitems.push_back(Item{(int32_t)fl[t], 0, 0, 0, 0, 0, 0, 0});
-    sadd(p.sbwd, S_BWD_FIRST, l, i0);
-    const i64 nblocks = (wmax + fc::SNB - 1) / fc::SNB;
-    for (i64 b = nblocks - 1; b >= 1; --b) {
-      const i64 c0 = b * fc::SNB;
-      i0 = (i64)p.sitems.size();
-      for (i64 t = 0; t < nl; ++t) {
-        const i64 f = fl[t];
-        if (s.f_w[f] <= c0) continue;
-        // the last column tile (the previous block's columns) also forms that block's solution
-        for (i64 j = 0; j < c0; j += fc::BCOLS)
-          p.sitems.push_back(Item{(int32_t)f, (int32_t)c0, (int32_t)j, j == c0 - fc::BCOLS ? 1 : 0, 0, 0, 0, 0});
-      }
-      sadd(p.sbwd, S_BWD_STEP, l, i0);
-    }
-  }
-  // one right-hand side: per level the gather, then the whole block chain in one launch; the
-  // backward's gather, below and first steps, then the chain. A front's forward workgroups are
-  // in increasing rows and its backward ones in decreasing blocks: each waits only on earlier ones.
-  for (i64 l = 0; l < s.levels; ++l) {
-    const i64* fl = &s.lvl_fronts[s.lvl_ptr[l]];
-    const i64 nl = s.lvl_ptr[l + 1] - s.lvl_ptr[l];
-    i64 i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t) p.sitems.push_back(Item{(int32_t)fl[t], 0, 0, 0, 0, 0, 0, 0});
-    sadd(p.sfwd1, S_GATHER, l, i0);
-    i0 = (i64)p.sitems.size();
-    bool chains = false;  // a front of several blocks: the launch forms block solutions
-    i64 tiles = 0;
-    for (i64 t = 0; t < nl; ++t) {
-      chains |= s.f_w[fl[t]] > fc::SNB;
-      tiles = std::max<i64>(tiles, (s.f_m[fl[t]] + fc::FROWS - 1) / fc::FROWS);
-    }
-    if (!chains) {  // one block a front: the step launch of the many-right-hand-side lists
-      for (i64 t = 0; t < nl; ++t) {
-        const i64 f = fl[t], c1 = s.f_w[f];
-        for (i64 r = c1; r < s.f_m[f]; r += fc::SROWS)
-          p.sitems.push_back(Item{(int32_t)f, 0, (int32_t)r, 0, 0, 0, 0, 0});
-      }
-      sadd(p.sfwd1, S_FWD_STEP, l, i0);
-      continue;
-    }
+    sadd(p.sfwd, S_FWD_ONE, l, i0);
     // tile-major across the level's fronts, the tiles of the fronts' own rows (the chains) first:
     // every chain starts in the first workgroups, and the tiles below, which only follow the
     // chains, never hold a slot a chain tile waits for
+    i0 = (i64)p.sitems.size();
+    i64 tiles = 0;
+    for (const i64 f : wide) tiles = std::max<i64>(tiles, (s.f_m[f] + fc::SNB - 1) / fc::SNB);
     for (int below = 0; below < 2; ++below)
       for (i64 k = 0; k < tiles; ++k)
-        for (i64 t = 0; t < nl; ++t) {
-          const i64 f = fl[t], c1 = std::min<i64>(fc::SNB, s.f_w[f]), r0 = k * fc::FROWS;
-          if ((r0 >= s.f_w[f]) != (below == 1)) continue;
-          if (r0 < s.f_m[f] && c1 < s.f_m[f] && r0 + fc::FROWS - 1 >= c1)  // a row of the tile below the first block
-            p.sitems.push_back(Item{(int32_t)f, (int32_t)r0, 0, 0, 0, 0, 0, 0});
-        }
-    sadd(p.sfwd1, S_FWD_FRONT, l, i0);
+        for (const i64 f : wide)
+          if ((k >= blocks(f)) == (below == 1) && k * fc::SNB < s.f_m[f]) sitem(f, k, 0);
+    sadd(p.sfwd, S_FWD, l, i0);
   }
   for (i64 l = s.levels - 1; l >= 0; --l) {
-    const i64* fl = &s.lvl_fronts[s.lvl_ptr[l]];
-    const i64 nl = s.lvl_ptr[l + 1] - s.lvl_ptr[l];
-    i64 i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t)
-      if (s.f_m[fl[t]] > s.f_w[fl[t]]) p.sitems.push_back(Item{(int32_t)fl[t], 0, 0, 0, 0, 0, 0, 0});
-    sadd(p.sbwd1, S_BWD_GATHER, l, i0);
-    i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t) {
-      const i64 f = fl[t];
-      if (s.f_m[f] == s.f_w[f]) continue;
-      for (i64 j = 0; j < s.f_w[f]; j += fc::SCOLS) p.sitems.push_back(Item{(int32_t)f, (int32_t)j, 0, 0, 0, 0, 0, 0});
+    sort_level(l);
+    // the products with the rows below of all but the one-block fronts with few of them
+    auto fused = [&](i64 f) { return blocks(f) <= 1 && s.f_m[f] - s.f_w[f] <= fc::BELOW_FUSE; };
+    i64 i0 = (i64)p.sitems.size(), count = 0;
+    for (i64 q = s.lvl_ptr[l]; q < s.lvl_ptr[l + 1]; ++q) {
+      const i64 f = s.lvl_fronts[q];
+      if (s.f_m[f] > s.f_w[f] && !fused(f)) count += (s.f_w[f] + 15) / 16;
     }
-    sadd(p.sbwd1, S_BWD_BELOW, l, i0);
+    const i64 cb = count < SOLVE_FEW ? 1 : 2;
+    for (i64 q = s.lvl_ptr[l]; q < s.lvl_ptr[l + 1]; ++q) {
+      const i64 f = s.lvl_fronts[q];
+      if (s.f_m[f] > s.f_w[f] && !fused(f))
+        for (i64 j = 0; j < s.f_w[f]; j += 16 * cb) sitem(f, j, 0);
+    }
+    sadd(p.sbwd, S_BELOW, l, i0, (int32_t)cb);
     i0 = (i64)p.sitems.size();
-    for (i64 t = 0; t < nl; ++t) p.sitems.push_back(Item{(int32_t)fl[t], 0, 0, 0, 0, 0, 0, 0});
-    sadd(p.sbwd1, S_BWD_FIRST, l, i0);
+    for (const i64 f : one) sitem(f, 0, fused(f));
+    sadd(p.sbwd, S_BWD_ONE, l, i0);
     // by distance from the front's last block, across the level's fronts: every chain starts in
     // the first workgroups, and a block's x is formed by an earlier workgroup than its users
     i0 = (i64)p.sitems.size();
     i64 depth = 0;
-    for (i64 t = 0; t < nl; ++t) depth = std::max<i64>(depth, (s.f_w[fl[t]] + fc::SNB - 1) / fc::SNB - 1);
+    for (const i64 f : wide) depth = std::max<i64>(depth, blocks(f));
     for (i64 k = 0; k < depth; ++k)
-      for (i64 t = 0; t < nl; ++t) {
-        const i64 f = fl[t], jb = (s.f_w[f] + fc::SNB - 1) / fc::SNB - 2 - k;
-        if (jb >= 0) p.sitems.push_back(Item{(int32_t)f, (int32_t)jb, 0, 0, 0, 0, 0, 0});
-      }
-    sadd(p.sbwd1, S_BWD_FRONT, l, i0);
+      for (const i64 f : wide)
+        if (k < blocks(f)) sitem(f, blocks(f) - 1 - k, fused(f));
+    sadd(p.sbwd, S_BWD, l, i0);
   }
   p.uoff.assign(s.f_soff.begin(), s.f_soff.end());
   p.u_solve = s.s_size;
@@ -717,12 +671,15 @@ struct DeviceStruct {
   int64_t* a_pos = nullptr;
   int64_t* diag_src = nullptr;
   int64_t* perm = nullptr;
+  uint32_t* gptr = nullptr;  // per front row: its entries in gsrc (rows of u that land on it)
+  uint32_t* gsrc = nullptr;
   ~DeviceStruct() {
     if (device < 0) return;
     int cur = 0;
     (void)hipGetDevice(&cur);
     (void)hipSetDevice(device);
-    for (void* q : {(void*)fronts, (void*)kids, (void*)rel, (void*)rows, (void*)a_pos, (void*)diag_src, (void*)perm})
+    for (void* q : {(void*)fronts, (void*)kids, (void*)rel, (void*)rows, (void*)a_pos, (void*)diag_src, (void*)perm,
+                    (void*)gptr, (void*)gsrc})
       dfree(q);
     (void)hipSetDevice(cur);
   }
@@ -741,6 +698,8 @@ struct DevicePlan {
   int64_t* a_pos = nullptr;
   int64_t* diag_src = nullptr;
   int64_t* perm = nullptr;
+  uint32_t* gptr = nullptr;
+  uint32_t* gsrc = nullptr;
   fc::Item* items = nullptr;
   fc::EaRange* earanges = nullptr;
   fc::GemmItem* gitems = nullptr;
@@ -829,6 +788,23 @@ struct fc_symbolic {
       ds->a_pos = dupload(S.a_pos, st);
       ds->diag_src = dupload(diag_src, st);
       ds->perm = dupload(S.perm, st);
+      // the solves' gather: for each front row, the rows of the children's contributions that land
+      // on it, child after child
+      std::vector<uint32_t> gptr((size_t)S.f_rptr[S.nf] + 1, 0);
+      auto each = [&](auto visit) {
+        for (i64 f = 0; f < S.nf; ++f)
+          for (i64 q = S.f_kptr[f]; q < S.f_kptr[f + 1]; ++q) {
+            const i64 c = S.f_kids[q], cmu = S.f_m[c] - S.f_w[c];
+            for (i64 i = 0; i < cmu; ++i) visit((size_t)(S.f_rptr[f] + S.rel[S.f_rel_off[c] + i]), S.f_soff[c] + i);
+          }
+      };
+      each([&](size_t row, i64) { ++gptr[row + 1]; });
+      for (size_t k = 1; k < gptr.size(); ++k) gptr[k] += gptr[k - 1];
+      std::vector<uint32_t> gsrc(gptr.back()), at(gptr.begin(), gptr.end() - 1);
+      each([&](size_t row, i64 src) { gsrc[at[row]++] = (uint32_t)src; });
+      ds->gptr = dupload(gptr, st);
+      ds->gsrc = dupload(gsrc, st);
+      HIP_CHECK(hipStreamSynchronize(st));
       structs.push_back(ds);
     }
     auto p = std::make_shared<DevicePlan>();
@@ -842,6 +818,8 @@ struct fc_symbolic {
     p->a_pos = ds->a_pos;
     p->diag_src = ds->diag_src;
     p->perm = ds->perm;
+    p->gptr = ds->gptr;
+    p->gsrc = ds->gsrc;
     p->items = dupload(pr->items, st);
     p->earanges = dupload(pr->earanges, st);
     p->gitems = dupload(pr->gitems, st);
@@ -1293,8 +1271,8 @@ int factor_host(fc_factor* F, const double* upper_val, uint64_t nnz, fc_error* e
   }
 }
 
-// A solve pass's device work: x and y (n x nr), the fronts' contributions, and the error word of
-// the one-right-hand-side chains (set when a wait gave up).
+// A solve pass's device work: x and y (n x nr, the right-hand sides of an equation side by side), the
+// fronts' contributions, and the error word of the chains (set when a wait gave up).
 struct SolveWork {
   double *xp, *yp, *u;
   int32_t* err;
@@ -1307,75 +1285,53 @@ int64_t solve_spin_limit() {
   return (int64_t)1 << 22;
 }
 
-template <typename T, int R>
-void run_solve_r(const fc_factor* F, const SolveWork& w, i64 ldx, int nrhs, hipStream_t st) {
-  const Program& prog = *F->prog;
+template <typename T, int NG>
+void run_solve_ng(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st) {
   DevicePlan& P = *F->plan;
   const T* L = (const T*)F->L;
   const T* Inv = (const T*)F->inv.p;
-  double *xp = w.xp, *yp = w.yp, *u = w.u;
-  int32_t* err = w.err;
   const int64_t limit = solve_spin_limit();
-  const int mark = R == 1;  // the chained passes: the gathers mark the block solutions to come
-  const int groups = (nrhs + fc::RSTEP - 1) / fc::RSTEP;  // block steps: right-hand-side groups
+  const int groups = (nr + fc::SRHS * NG - 1) / (fc::SRHS * NG);
   auto run = [&](const fc::Launch& l) {
     const fc::Item* it = P.sitems + l.item0;
-    dim3 g(l.count), b(256);
+    const dim3 g((unsigned)l.count * groups), b(fc::STHREADS), b1(fc::ONE_THREADS);
     switch (l.kind) {
-      case S_GATHER:
-        fc::k_fwd_gather<T, R><<<g, b, 0, st>>>(it, P.fronts, P.kids, P.rel, Inv, xp, yp, ldx, nrhs, u, P.uoff, mark);
+      case S_FWD:
+        fc::k_fwd<T, NG><<<g, b, 0, st>>>(it, P.fronts, P.gptr, P.gsrc, L, Inv, w.xp, w.yp, w.u, P.uoff, nr, l.count,
+                                          w.err, limit);
         break;
-      case S_FWD_STEP:  // every right-hand side in one workgroup (groups side by side would each
-                        // read the step's rows of L again: measured slower)
-        fc::k_fwd_step<T, R><<<g, b, 0, st>>>(it, P.fronts, L, Inv, xp, yp, ldx, nrhs, u, P.uoff, l.count);
+      case S_FWD_ONE:
+        fc::k_fwd_one<T, NG><<<g, b1, 0, st>>>(it, P.fronts, P.gptr, P.gsrc, L, Inv, w.xp, w.yp, w.u, P.uoff, nr, l.count);
         break;
-      case S_BWD_GATHER:
-        fc::k_bwd_gather<<<g, b, 0, st>>>(it, P.fronts, P.rows, xp, ldx, nrhs, u, P.uoff);
+      case S_BELOW:
+        if (l.pad == 1) fc::k_bwd_below<T, NG, 1><<<g, b, 0, st>>>(it, P.fronts, L, P.rows, w.xp, w.yp, nr, l.count);
+        else fc::k_bwd_below<T, NG, 2><<<g, b, 0, st>>>(it, P.fronts, L, P.rows, w.xp, w.yp, nr, l.count);
         break;
-      case S_BWD_BELOW:
-        fc::k_bwd_below<T, R><<<g, b, 0, st>>>(it, P.fronts, L, u, P.uoff, yp, ldx, nrhs);
+      case S_BWD:
+        fc::k_bwd<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, P.rows, w.yp, w.xp, nr, l.count, w.err, limit);
         break;
-      case S_BWD_FIRST:
-        fc::k_bwd_first<T, R><<<g, b, 0, st>>>(it, P.fronts, Inv, yp, xp, ldx, nrhs, mark);
-        break;
-      case S_BWD_STEP:
-        if constexpr (R == 1) fc::k_bwd_step1<T><<<g, b, 0, st>>>(it, P.fronts, L, Inv, yp, xp);
-        else  // several right-hand sides: groups of RSTEP side by side (a step's tile is small)
-          fc::k_bwd_step<T, fc::RSTEP><<<dim3(l.count * groups), b, 0, st>>>(it, P.fronts, L, Inv, yp, xp, ldx, nrhs,
-                                                                             l.count);
-        break;
-      case S_FWD_FRONT:
-        fc::k_fwd_front<T><<<g, b, fc::SNB * fc::SNB * sizeof(T), st>>>(it, P.fronts, L, Inv, xp, yp, u, P.uoff, err,
-                                                                         limit);
-        break;
-      case S_BWD_FRONT:
-        fc::k_bwd_front<T><<<g, b, 0, st>>>(it, P.fronts, L, Inv, yp, xp, err, limit);
+      case S_BWD_ONE:
+        fc::k_bwd_one<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, P.rows, w.yp, w.xp, nr, l.count);
         break;
     }
   };
-  if constexpr (R == 1) {
-    for (const fc::Launch& l : prog.sfwd1) run(l);
-    for (const fc::Launch& l : prog.sbwd1) run(l);
-  } else {
-    for (const fc::Launch& l : prog.sfwd) run(l);
-    for (const fc::Launch& l : prog.sbwd) run(l);
-  }
+  for (const fc::Launch& l : F->prog->sfwd) run(l);
+  for (const fc::Launch& l : F->prog->sbwd) run(l);
   HIP_CHECK(hipGetLastError());
 }
 
 template <typename T>
-void run_solve(const fc_factor* F, const SolveWork& w, i64 ldx, int nrhs, hipStream_t st) {
-  if (nrhs == 1) run_solve_r<T, 1>(F, w, ldx, nrhs, st);
-  else if (nrhs <= fc::RC / 2) run_solve_r<T, fc::RC / 2>(F, w, ldx, nrhs, st);  // a Lanczos block
-  else run_solve_r<T, fc::RC>(F, w, ldx, nrhs, st);
+void run_solve(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st) {
+  if (nr <= fc::SRHS) run_solve_ng<T, 1>(F, w, nr, st);
+  else run_solve_ng<T, 2>(F, w, nr, st);
 }
 
 // The solve's launches for nr right-hand sides in w, replayed from a hipGraph when
 // opts.use_graph asks for it (bit 1): captured on first use for each (nr, workspaces).
-void solve_launches(const fc_factor* F, const SolveWork& w, i64 n, int nr, hipStream_t st) {
+void solve_launches(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st) {
   auto eager = [&]() {
-    if (F->precision == FC_FP64) run_solve<double>(F, w, n, nr, st);
-    else run_solve<float>(F, w, n, nr, st);
+    if (F->precision == FC_FP64) run_solve<double>(F, w, nr, st);
+    else run_solve<float>(F, w, nr, st);
   };
   if (!(F->opts.use_graph & 2)) return eager();
   for (const auto& sg : F->sgraphs)
@@ -1428,9 +1384,9 @@ void solve_device(const fc_factor* F, double* b, i64 n, int nrhs, i64 ldb, hipSt
     w.yp = (double*)F->yp.get((size_t)n * nr * sizeof(double));
     w.u = (double*)F->usolve.get((size_t)std::max<i64>(F->prog->u_solve * nr, 1) * sizeof(double));
     w.err = err;
-    fc::k_permute<<<blocks_for(n), 256, 0, st>>>(br, w.xp, F->plan->perm, n, nr, ldb, n, 0);
-    solve_launches(F, w, n, nr, st);
-    fc::k_permute<<<blocks_for(n), 256, 0, st>>>(w.xp, br, F->plan->perm, n, nr, n, ldb, 1);
+    fc::k_solve_in<<<blocks_for(n * nr), 256, 0, st>>>(br, w.xp, w.yp, F->plan->perm, n, nr, ldb);
+    solve_launches(F, w, nr, st);
+    fc::k_solve_out<<<blocks_for(n * nr), 256, 0, st>>>(w.xp, br, F->plan->perm, n, nr, ldb);
   }
   HIP_CHECK(hipGetLastError());
   solve_check(err, st);
@@ -3146,10 +3102,10 @@ int fc_solve_device_noalloc(const fc_factor* f, double* b, uint64_t n, uint64_t 
       w.yp = (double*)(base + align256((size_t)n * nr * sizeof(double)));
       w.u = (double*)(base + 2 * align256((size_t)n * nr * sizeof(double)));
       w.err = serr;
-      fc::k_permute<<<blocks_for((i64)n), 256, 0, st>>>(br, w.xp, f->plan->perm, (i64)n, nr, (i64)ldb, (i64)n, 0);
-      if (f->precision == FC_FP64) run_solve<double>(f, w, (i64)n, nr, st);  // eager: no graph
-      else run_solve<float>(f, w, (i64)n, nr, st);
-      fc::k_permute<<<blocks_for((i64)n), 256, 0, st>>>(w.xp, br, f->plan->perm, (i64)n, nr, (i64)n, (i64)ldb, 1);
+      fc::k_solve_in<<<blocks_for((i64)n * nr), 256, 0, st>>>(br, w.xp, w.yp, f->plan->perm, (i64)n, nr, (i64)ldb);
+      if (f->precision == FC_FP64) run_solve<double>(f, w, nr, st);  // eager: no graph
+      else run_solve<float>(f, w, nr, st);
+      fc::k_solve_out<<<blocks_for((i64)n * nr), 256, 0, st>>>(w.xp, br, f->plan->perm, (i64)n, nr, (i64)ldb);
     }
     HIP_CHECK(hipGetLastError());
     solve_check(serr, st);
