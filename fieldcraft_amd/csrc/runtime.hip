@@ -1893,11 +1893,16 @@ struct LanczosWork {
   i64 cap;
   double *Q = nullptr, *MQ = nullptr, *W = nullptr, *MW = nullptr, *part = nullptr, *C = nullptr;
   int64_t* at = nullptr;
-  int chunks = 1;
+  int chunks = 1;       // argmax chunks (TS_ROWS rows)
+  i64 drows = 1;        // rows of a partial sum of the dot products, and their number
+  int dchunks = 1;
+  double* pinned = nullptr;  // PINNED host values the dot products' sums are written to as well
+  static constexpr int PINNED = 1024;
   std::vector<double> host;
 
   ~LanczosWork() {
     for (void* p : {(void*)Q, (void*)MQ, (void*)W, (void*)MW, (void*)part, (void*)C, (void*)at}) dfree(p);
+    if (pinned) (void)hipHostFree(pinned);
   }
   double* q(i64 j) { return Q + j * n; }
   double* mq(i64 j) { return MQ + j * n; }
@@ -1905,16 +1910,29 @@ struct LanczosWork {
   void mass(const double* x, double* y, int k) {
     fc::k_spmm<<<blocks_for(n * 8), 256, 0, st>>>(n, M->ptr, M->idx, M->val, x, y, k, n);
   }
-  // host C (m x b, row-major) = A^T B: A n x m (leading dimension n), B n x b
+  // C (m x b, row-major, device) = A^T B: A n x m (leading dimension n), B n x b; out (pinned, or
+  // null) gets a copy that the host may read after the next synchronization.
+  void dots_device(const double* A, int m, const double* B, int b, double* out) {
+    if (m == 0 || b == 0) return;
+    dim3 grid(dchunks, (m + fc::TS_COLS - 1) / fc::TS_COLS);
+    fc::k_ts_dots<<<grid, 256, 0, st>>>(n, drows, A, n, m, B, n, b, part);
+    fc::k_ts_dots_sum<<<(m * b + 63) / 64, 64, 0, st>>>(part, dchunks, m, b, C, out);
+  }
+  // the same for at most TS_MAXB columns of A, on the host
   const std::vector<double>& dots(const double* A, int m, const double* B, int b) {
-    host.assign((size_t)m * b, 0.0);
-    if (m == 0 || b == 0) return host;
-    dim3 grid(chunks, (m + fc::TS_COLS - 1) / fc::TS_COLS);
-    fc::k_ts_dots<<<grid, 256, 0, st>>>(n, A, n, m, B, n, b, part);
-    fc::k_ts_dots_sum<<<(m * b + 255) / 256, 256, 0, st>>>(part, chunks, m, b, C);
-    HIP_CHECK(hipMemcpyAsync(host.data(), C, sizeof(double) * m * b, hipMemcpyDeviceToHost, st));
+    dots_device(A, m, B, b, pinned);
     HIP_CHECK(hipStreamSynchronize(st));
+    host.assign(pinned, pinned + (size_t)m * b);
     return host;
+  }
+  // B = beta B + alpha A C for b columns with the C that dots_device left (in pieces the update
+  // kernel's LDS holds)
+  void update_device(const double* A, int m, double* B, int b, double alpha, double beta) {
+    const int per = std::max(1, fc::TS_MAXC / std::max(b, 1));
+    for (int i0 = 0; i0 < m; i0 += per)
+      fc::k_ts_update<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, A + (i64)i0 * n, n, std::min(per, m - i0),
+                                                                    C + (size_t)i0 * b, b, B, n, b, alpha,
+                                                                    i0 == 0 ? beta : 1.0);
   }
   // B = beta B + alpha A c for b columns; c host m x b row-major (uploaded in pieces the
   // update kernel's LDS holds)
@@ -1932,7 +1950,10 @@ struct LanczosWork {
     }
   }
   void scale(double* x, double s) { fc::k_scale<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, x, s); }
-  void copy(const double* x, double* y) { fc::k_copy_col<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, x, y); }
+  // q = s v, mv = s mv
+  void normalize(const double* v, double* q, double* mv, double s) {
+    fc::k_normalize<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, v, q, mv, s);
+  }
   double mnorm2(const double* x, const double* mx) { return std::max(dots(x, 1, mx, 1)[0], 0.0); }
   void random_into(double* x, XorShift& rng) {
     std::vector<double> v(n);
@@ -1952,15 +1973,17 @@ struct LanczosWork {
 int orthonormalize_block(LanczosWork& L, int k, i64 mb, XorShift& rng, std::vector<double>& r) {
   r.assign((size_t)k * k, 0.0);
   L.mass(L.W, L.MW, k);
-  std::vector<double> before(k);
-  {
-    const std::vector<double>& g = L.dots(L.W, k, L.MW, k);
-    for (int i = 0; i < k; ++i) before[i] = std::sqrt(std::max(g[(size_t)i * k + i], 0.0));
-  }
-  auto project_basis = [&](double* w, int cols) {
+  // The coefficients go from the dot products to the update on the device; the host reads its copies
+  // (the squared norms before, then each column's coefficients and its norm after) where a column's
+  // norm has to be judged: one synchronization a column.
+  const double* gram = L.pinned;  // k x k
+  double* cols = L.pinned + (size_t)k * k;
+  static_assert(LanczosWork::PINNED >= fc::TS_MAXB * fc::TS_MAXB + 2 * fc::TS_MAXB + 1, "pinned values of a column");
+  L.dots_device(L.W, k, L.MW, k, L.pinned);
+  auto project_basis = [&](double* w, int nc) {
     for (int pass = 0; pass < 2 && mb > 0; ++pass) {
-      const std::vector<double> c = L.dots(L.MQ, (int)mb, w, cols);
-      L.update(L.Q, (int)mb, c, w, cols, -1.0, 1.0);
+      L.dots_device(L.MQ, (int)mb, w, nc, nullptr);
+      L.update_device(L.Q, (int)mb, w, nc, -1.0, 1.0);
     }
   };
   project_basis(L.W, k);
@@ -1968,27 +1991,33 @@ int orthonormalize_block(LanczosWork& L, int k, i64 mb, XorShift& rng, std::vect
   for (int i = 0; i < k; ++i) {
     double* v = L.W + (i64)i * L.n;
     bool fresh = false;
+    double before = 0.0;
     for (int attempt = 0; attempt < 4; ++attempt) {
       if (fresh) {
         L.random_into(v, rng);
         L.mass(v, L.MW, 1);
-        before[i] = std::sqrt(L.mnorm2(v, L.MW));
+        L.dots_device(v, 1, L.MW, 1, cols);
+        HIP_CHECK(hipStreamSynchronize(L.st));
+        before = std::sqrt(std::max(cols[0], 0.0));
         project_basis(v, 1);
       }
       for (int pass = 0; pass < 2 && kept > 0; ++pass) {
-        const std::vector<double> c = L.dots(L.mq(mb), kept, v, 1);
-        L.update(L.q(mb), kept, c, v, 1, -1.0, 1.0);
-        if (!fresh)
-          for (int j = 0; j < kept; ++j) r[(size_t)j * k + i] += c[j];
+        L.dots_device(L.mq(mb), kept, v, 1, cols + 1 + pass * kept);
+        L.update_device(L.q(mb), kept, v, 1, -1.0, 1.0);
       }
       double* mv = L.mq(mb + kept);
       L.mass(v, mv, 1);
-      const double norm = std::sqrt(L.mnorm2(v, mv));
-      if (norm > 1e-8 * before[i] && norm > 0.0) {
+      L.dots_device(v, 1, mv, 1, cols);
+      HIP_CHECK(hipStreamSynchronize(L.st));
+      const double norm = std::sqrt(std::max(cols[0], 0.0));
+      if (!fresh) {
+        before = std::sqrt(std::max(gram[(size_t)i * k + i], 0.0));
+        for (int pass = 0; pass < 2; ++pass)
+          for (int j = 0; j < kept; ++j) r[(size_t)j * k + i] += cols[1 + pass * kept + j];
+      }
+      if (norm > 1e-8 * before && norm > 0.0) {
         if (!fresh) r[(size_t)i * k + i] = norm;
-        L.copy(v, L.q(mb + kept));
-        L.scale(L.q(mb + kept), 1.0 / norm);
-        L.scale(mv, 1.0 / norm);
+        L.normalize(v, L.q(mb + kept), mv, 1.0 / norm);
         ++kept;
         break;
       }
@@ -2018,7 +2047,15 @@ LanczosResult lanczos_run(i64 n, const std::function<void(double*, int)>& solve,
   L.MQ = dalloc<double>((size_t)n * cap);
   L.W = dalloc<double>((size_t)n * fc::TS_MAXB);
   L.MW = dalloc<double>((size_t)n * fc::TS_MAXB);
-  L.part = dalloc<double>((size_t)L.chunks * cap * fc::TS_MAXB);
+  L.drows = fc::ts_rows(n);
+  L.dchunks = (int)std::max<i64>(1, (n + L.drows - 1) / L.drows);
+  L.part = dalloc<double>((size_t)L.dchunks * cap * fc::TS_MAXB);
+  if (void* h = nullptr; hipHostMalloc(&h, LanczosWork::PINNED * sizeof(double), hipHostMallocDefault) == hipSuccess) {
+    L.pinned = (double*)h;
+  } else {
+    (void)hipGetLastError();
+    throw std::bad_alloc();
+  }
   L.C = dalloc<double>((size_t)std::max<i64>(cap * fc::TS_MAXB, fc::TS_MAXC));
   L.at = dalloc<int64_t>((size_t)L.chunks);
   XorShift rng(0x9E3779B97F4A7C15ULL);
