@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace fc {
 
@@ -90,36 +91,30 @@ constexpr int LDL_YC = 16;   // target columns of one update window (and one til
 constexpr int LDL_KC = 128;  // source columns of Y staged in LDS at a time
 constexpr int LDL_PP = 8;    // pairs per thread per batch
 
+// The first position of the rising map rel[0, hi) with rel[i] >= v.
+__device__ __forceinline__ int ldl_first_at_least(const int32_t* __restrict__ rel, int hi, int64_t v) {
+  int lo = 0;
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (rel[mid] < v) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
 // own(rel(i), rel(c)) -= sum_{k < kw} L(p + i, k0 + k) Y(p + c, k), Y = L D (products and
-// subtract, cholesky.rs:531-686 with pivots), for c < min(wu, mu), c <= i < mu, restricted to the
-// target columns rel(c) in [cb, ce) (at most LDL_YC of them) and the target rows rel(i) in
-// [rb, re): each (i, c) summed by one thread in k order from 0.0. The window's Y entries are
-// staged in LDS LDL_KC columns at a time; each thread carries LDL_PP sums across the stages.
+// subtract, cholesky.rs:531-686 with pivots), for c in [ca, cz) (at most LDL_YC of them) and i in
+// [max(c, ia), iz): each (i, c) summed by one thread in k order from 0.0. rel null: rel(i) = rel0 + i.
+// The window's Y entries are staged in LDS LDL_KC columns at a time; each thread carries LDL_PP sums
+// across the stages, KU columns' loads of all of them in flight at a time (the sums themselves are
+// chains; one sum after the other, four loads at a time, waited on memory 8 kw / 4 times).
 // All threads of the workgroup call it together.
 template <typename T>
 __device__ inline void ldl_update(T* own, int64_t m, const T* lk, int64_t mk, int64_t k0, int kw,
-                                  const int8_t* pk, int64_t p, int64_t mu, int64_t wu, const int32_t* rel, bool rel_id,
-                                  int64_t rel0, int64_t cb, int64_t ce, int64_t rb, int64_t re) {
+                                  const int8_t* pk, int64_t p, const int32_t* rel, int64_t rel0, int64_t ca, int64_t cz,
+                                  int64_t ia, int64_t iz) {
 #pragma clang fp contract(off)
-  const int64_t cols = wu < mu ? wu : mu;
-  // the columns c whose target lies in [cb, ce) and the rows i whose target lies in [rb, re):
-  // rel is increasing, so both are ranges
-  auto first_at_least = [&](int64_t v, int64_t hi) {
-    if (rel_id) {
-      const int64_t t = v - rel0;
-      return t < 0 ? (int64_t)0 : (t > hi ? hi : t);
-    }
-    int64_t lo = 0;
-    while (lo < hi) {
-      const int64_t mid = (lo + hi) / 2;
-      if (rel[mid] < v) lo = mid + 1;
-      else hi = mid;
-    }
-    return lo;
-  };
-  const int64_t ca = first_at_least(cb, cols), cz = first_at_least(ce, cols);
-  const int64_t ia = first_at_least(rb, mu), iz = first_at_least(re, mu);
-  if (ca >= cz || ia >= iz) return;
+  constexpr int KU = sizeof(T) == 8 ? 4 : 2;
   const int ncol = (int)(cz - ca);
   // pairs of column ca + t: rows max(ca + t, ia) .. iz; pre[t] = pairs before it
   __shared__ int64_t pre[LDL_YC + 1];
@@ -145,7 +140,7 @@ __device__ inline void ldl_update(T* own, int64_t m, const T* lk, int64_t mk, in
       const int64_t q = q0 + threadIdx.x + (int64_t)t * blockDim.x;
       sum[t] = T{};
       yrow[t] = -1;
-      li[t] = 0;
+      li[t] = d0 + p + ca - k0;  // (no pair: any entry of the column)
       tgt[t] = 0;
       if (q < pairs) {
         int c = 0;
@@ -154,10 +149,11 @@ __device__ inline void ldl_update(T* own, int64_t m, const T* lk, int64_t mk, in
         const int64_t i = lo + (q - pre[c]);
         yrow[t] = c;
         li[t] = d0 + p + i - k0;  // L(p + i, k0)
-        const int64_t ri = rel_id ? rel0 + i : rel[i], rc = rel_id ? rel0 + ca + c : rel[ca + c];
+        const int64_t ri = rel ? rel[i] : rel0 + i, rc = rel ? rel[ca + c] : rel0 + ca + c;
         tgt[t] = ldl_offset(m, rc) + ri - rc;
       }
     }
+    int64_t off = 0;  // entries from column k0's to column k0 + kb + kk's
     for (int kb = 0; kb < kw; kb += LDL_KC) {
       const int kn = kw - kb < LDL_KC ? kw - kb : LDL_KC;
       __syncthreads();  // the previous stage is consumed
@@ -179,26 +175,31 @@ __device__ inline void ldl_update(T* own, int64_t m, const T* lk, int64_t mk, in
         ys[t * LDL_KC + kk] = y;
       }
       __syncthreads();
+      // whole batches with no test inside (a test would move each load behind it)
+      auto batch = [&](int k1, auto nb) {
+        constexpr int NB_ = decltype(nb)::value;
+        T l[NB_][LDL_PP];
 #pragma unroll
-      for (int t = 0; t < LDL_PP; ++t) {
-        if (yrow[t] < 0) continue;
-        const T* yv = ys + yrow[t] * LDL_KC;
-        int64_t at = li[t];
-        T acc = sum[t];
-        int64_t step = mk - k0 - kb - 1;  // entries of column k0 + k + 1 lie mk - k0 - k - 1 on
-#pragma unroll 4
-        for (int kk = 0; kk < kn; ++kk) {
-          acc += lk[at] * yv[kk];
-          at += step;
-          step -= 1;
+        for (int u = 0; u < NB_; ++u) {  // column k0 + k + 1's entry lies mk - k0 - k - 1 on
+#pragma unroll
+          for (int t = 0; t < LDL_PP; ++t) l[u][t] = lk[li[t] + off];
+          off += mk - k0 - kb - (k1 + u) - 1;
         }
-        sum[t] = acc;
-        li[t] = at;
-      }
+#pragma unroll
+        for (int u = 0; u < NB_; ++u)
+#pragma unroll
+          for (int t = 0; t < LDL_PP; ++t) sum[t] += l[u][t] * ys[max(yrow[t], 0) * LDL_KC + k1 + u];
+      };
+      int k1 = 0;
+      for (; k1 + KU <= kn; k1 += KU) batch(k1, std::integral_constant<int, KU>{});
+      for (; k1 < kn; ++k1) batch(k1, std::integral_constant<int, 1>{});
     }
+    T old[LDL_PP];
+#pragma unroll
+    for (int t = 0; t < LDL_PP; ++t) old[t] = yrow[t] >= 0 ? own[tgt[t]] : T{};
 #pragma unroll
     for (int t = 0; t < LDL_PP; ++t)
-      if (yrow[t] >= 0) own[tgt[t]] -= sum[t];
+      if (yrow[t] >= 0) own[tgt[t]] = old[t] - sum[t];
   }
   __syncthreads();
 }
@@ -222,7 +223,8 @@ __global__ void k_ldlt_zero(int64_t n, T* __restrict__ v) {
 // The descendants' updates of the supernodes of one level (the assemble of cholesky.rs:1069-1124
 // with Y = L D): workgroup t takes the target columns [tiles[t].b, tiles[t].e) of supernode
 // tiles[t].j and applies every update to them in order, so each entry receives its updates in
-// the reference's order whatever the tiling.
+// the reference's order whatever the tiling. The ranges of 64 updates at a time are found side by side,
+// a thread a bound (one update after the other, each search was a chain of its own).
 struct LdlTile {
   int64_t j, b, e;  // supernode, target columns [b, e)
   int64_t rb, re;   // target rows [rb, re)
@@ -232,15 +234,66 @@ __global__ __launch_bounds__(256) void k_ldlt_assemble(const LdlTile* __restrict
                                                        const LdlUpdate* __restrict__ U, const int32_t* __restrict__ rel,
                                                        T* __restrict__ val, const int8_t* __restrict__ piv) {
 #pragma clang fp contract(off)
+  constexpr int NU = 64;  // updates whose ranges are found together
+  __shared__ int range[NU][4];
   const LdlTile tl = tiles[blockIdx.x];
   const LdlSupernode J = S[tl.j];
   T* own = val + J.voff;
-  for (int64_t u = J.upd0; u < J.upd1; ++u) {
-    const LdlUpdate up = U[u];
-    const LdlSupernode K = S[up.k];
-    ldl_update(own, J.m, val + K.voff, K.m, 0, K.w, piv + K.first, up.p1, K.m - up.p1, up.p2 - up.p1, rel + up.rel, false,
-               0, tl.b, tl.e, tl.rb, tl.re);
+  for (int64_t u0 = J.upd0; u0 < J.upd1; u0 += NU) {
+    __syncthreads();
+    {  // thread (update, bound): the columns c and rows i of the update that land in the tile
+      const int t = threadIdx.x >> 2, which = threadIdx.x & 3;
+      int at = 0;
+      if (u0 + t < J.upd1) {
+        const LdlUpdate up = U[u0 + t];
+        const int mu = S[up.k].m - up.p1, wu = up.p2 - up.p1;
+        at = ldl_first_at_least(rel + up.rel, which < 2 && wu < mu ? wu : mu,
+                                which == 0 ? tl.b : (which == 1 ? tl.e : (which == 2 ? tl.rb : tl.re)));
+      }
+      range[t][which] = at;
+    }
+    __syncthreads();
+    for (int t = 0; t < NU; ++t) {
+      const int ca = range[t][0], cz = range[t][1], ia = range[t][2], iz = range[t][3];
+      if (ca >= cz || ia >= iz) continue;  // (an update past the last has an empty range)
+      const LdlUpdate up = U[u0 + t];
+      const LdlSupernode K = S[up.k];
+      ldl_update(own, J.m, val + K.voff, K.m, 0, K.w, piv + K.first, up.p1, rel + up.rel, 0, ca, cz, ia, iz);
+    }
   }
+}
+
+// The largest of a wave's values and the smallest of its integers: permutations within rows of 16
+// lanes (no LDS round trip), then the four rows' by scalar reads.
+template <int CTRL>
+__device__ __forceinline__ int ldl_dpp(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double ldl_dpp(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)ldl_dpp<CTRL>((int)(uint32_t)b), hi = (uint32_t)ldl_dpp<CTRL>((int)(uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double ldl_lane(double v, int l) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, l), hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double ldl_wave_max(double v) {
+  v = fmax(v, ldl_dpp<0xB1>(v));   // lane ^ 1
+  v = fmax(v, ldl_dpp<0x4E>(v));   // lane ^ 2
+  v = fmax(v, ldl_dpp<0x141>(v));  // the half row's mirror
+  v = fmax(v, ldl_dpp<0x140>(v));  // the row's mirror
+  return fmax(fmax(ldl_lane(v, 0), ldl_lane(v, 16)), fmax(ldl_lane(v, 32), ldl_lane(v, 48)));
+}
+__device__ __forceinline__ int ldl_wave_min(int v) {
+  v = min(v, ldl_dpp<0xB1>(v));
+  v = min(v, ldl_dpp<0x4E>(v));
+  v = min(v, ldl_dpp<0x141>(v));
+  v = min(v, ldl_dpp<0x140>(v));
+  return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
 // One supernode per workgroup (supernode list sn[blockIdx.x]), assembled: the panels
@@ -280,86 +333,91 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
   T* A = m <= lds_rows ? reinterpret_cast<T*>(ldl_dyn) : work + J.scratch;
   T* B = A + m;
   const double* sc = scale + J.first;
-  __shared__ double red_v[16];   // one entry per wave (up to 1024 threads)
-  __shared__ int64_t red_i[16], red_n[16];
-  __shared__ int64_t sh[6];          // decisions broadcast by thread 0
-  __shared__ double shd[2];
+  __shared__ double red_v[2][16];   // one entry per wave (up to 1024 threads), two calls' worth
+  __shared__ int red_i[2][16], red_n[2][16];
+  int par = 0;
   int twos = 0;
+  // D of the panel's finished columns: kinds, D(q, q) and D(q + 1, q)
+  __shared__ int8_t pk[LDL_PANEL + 2];
+  __shared__ T d1[LDL_PANEL + 2], d2[LDL_PANEL + 2];
   // current(c) into out: column c rows k..m less the panel's factored columns c0..k (ldlt.rs:176-193)
   __shared__ T ydc[LDL_PANEL + 2];
   auto current = [&](int64_t c0, int64_t k, int64_t c, T* out) {
+    const int n = (int)(k - c0);
     auto row = [&](int q) { return LDL_AT(own, m, c, c0 + q); };
-    for (int64_t q = threadIdx.x; q < k - c0; q += blockDim.x)
-      ydc[q] = times_d_at(row, own, m, c0, pv + c0, (int)q, (int)(k - c0));
+    if ((int)threadIdx.x < n) {  // times_d (cholesky.rs:460-484) of row c, as times_d_at
+      const int q = threadIdx.x;
+      const T a = row(q), lo = row(q > 0 ? q - 1 : 0), hi = row(q + 1 < n ? q + 1 : q);
+      T y;
+      if (pk[q] == PIV_FIRST) y = a * d1[q] + (q + 1 < n ? hi : T{}) * d2[q];
+      else if (pk[q] == PIV_SECOND && q > 0 && pk[q - 1] == PIV_FIRST) y = lo * d2[q - 1] + a * d1[q];
+      else y = a * d1[q];
+      ydc[q] = y;
+    }
     __syncthreads();
+    constexpr int QB = sizeof(T) == 8 ? 16 : 8;  // columns in flight at a time
     const int64_t o0 = ldl_offset(m, c0) - c0;
     for (int64_t r = k + threadIdx.x; r < m; r += blockDim.x) {
       T v = r >= c ? LDL_AT(own, m, r, c) : LDL_AT(own, m, c, r);
-      int64_t o = o0 + r;  // (r, q): the next column's entry lies m - q - 1 on
-#pragma unroll 8
-      for (int64_t q = c0; q < k; ++q) {
-        v -= own[o] * ydc[q - c0];
-        o += m - q - 1;
-      }
+      int64_t o = o0 + r;  // (r, q): the next column's entry lies m - c0 - q - 1 on
+      // whole batches with no test inside (a test would move each load behind it)
+      auto batch = [&](int q0, auto nb) {
+        constexpr int NB_ = decltype(nb)::value;
+        T l[NB_];
+#pragma unroll
+        for (int j = 0; j < NB_; ++j) {
+          l[j] = own[o];
+          o += m - c0 - (q0 + j) - 1;
+        }
+#pragma unroll
+        for (int j = 0; j < NB_; ++j) v -= l[j] * ydc[q0 + j];
+      };
+      int q0 = 0;
+      for (; q0 + QB <= n; q0 += QB) batch(q0, std::integral_constant<int, QB>{});
+      for (; q0 + 4 <= n; q0 += 4) batch(q0, std::integral_constant<int, 4>{});
+      for (; q0 < n; ++q0) batch(q0, std::integral_constant<int, 1>{});
       out[r] = v;
     }
     __syncthreads();
   };
   // largest |v[i]| over [lo, hi) except skip (ldlt.rs:149-164): the first index of the largest,
-  // or the first NaN's index with NaN
+  // or the first NaN's index with NaN. Each wave reduces its own values by lane permutations within
+  // rows of 16 lanes; after one barrier every wave reduces the waves' results for itself.
   auto largest = [&](const T* v, int64_t lo, int64_t hi, int64_t skip, int64_t* at, double* value) {
+    constexpr int NONE32 = 0x7fffffff;
     double bv = 0.0;
-    int64_t bi = -1, nan_i = -1;
+    int bi = NONE32, bn = NONE32;
     for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
       if (i == skip) continue;
       const double x = ldl_mod(v[i]);
       if (isnan(x)) {
-        if (nan_i < 0) nan_i = i;
+        bn = min(bn, (int)i);
       } else if (x > bv) {
         bv = x;
-        bi = i;
+        bi = (int)i;
       }
     }
-    // the wave's best (largest value, then the lowest index; zeros carry no index) and first
-    // NaN, then thread 0 over the waves in order
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const double ov = __shfl_xor(bv, off, 64);
-      const int64_t oi = __shfl_xor(bi, off, 64), on = __shfl_xor(nan_i, off, 64);
-      if (ov > bv || (ov == bv && ov > 0.0 && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
-      if (on >= 0 && (nan_i < 0 || on < nan_i)) nan_i = on;
-    }
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const double wb = ldl_wave_max(bv);
+    const int wi = ldl_wave_min(bv == wb && bv > 0.0 ? bi : NONE32);
+    const int wn = __any(bn != NONE32) ? ldl_wave_min(bn) : NONE32;
     if (lane == 0) {
-      red_v[wv] = bv;
-      red_i[wv] = bi;
-      red_n[wv] = nan_i;
+      red_v[par][wv] = wb;
+      red_i[par][wv] = wi;
+      red_n[par][wv] = wn;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      int64_t best_i = -1, first_nan = -1;
-      double best = 0.0;
-      for (int t = 0; t < (int)(blockDim.x >> 6); ++t) {
-        if (red_v[t] > best || (red_v[t] == best && red_v[t] > 0.0 && red_i[t] < best_i)) {
-          best = red_v[t];
-          best_i = red_i[t];
-        }
-        if (red_n[t] >= 0 && (first_nan < 0 || red_n[t] < first_nan)) first_nan = red_n[t];
-      }
-      sh[4] = best_i < 0 ? lo : best_i;
-      shd[0] = best;
-      if (first_nan >= 0) {  // the reference returns at the first NaN it meets, whatever came before
-        sh[4] = first_nan;
-        shd[0] = __builtin_nan("");
-      }
+    const double rv = lane < nw ? red_v[par][lane] : 0.0;
+    const int ri = lane < nw ? red_i[par][lane] : NONE32, rn = lane < nw ? red_n[par][lane] : NONE32;
+    par ^= 1;  // the next call's slots: a wave may be there while another still reads these
+    const double best = ldl_wave_max(rv);
+    const int best_i = ldl_wave_min(rv == best && rv > 0.0 ? ri : NONE32), first_nan = ldl_wave_min(rn);
+    *at = best_i == NONE32 ? lo : best_i;
+    *value = best;
+    if (first_nan != NONE32) {  // the reference returns at the first NaN it meets, whatever came before
+      *at = first_nan;
+      *value = __builtin_nan("");
     }
-    __syncthreads();
-    *at = sh[4];
-    *value = shd[0];
-    __syncthreads();
   };
   auto bswap = [&](int64_t p, int64_t q) {
     if (p == q) return;
@@ -411,6 +469,7 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
     const int64_t end = c0 + LDL_PANEL < w ? c0 + LDL_PANEL : w;
     int64_t k = c0;
     while (k < end) {
+      const double sk = sc[od[k]];  // the row's scale if the pivot stays in place, loaded ahead
       current(c0, k, k, A);
       const double akk = ldl_mod(A[k]);
       int64_t r0;
@@ -461,7 +520,7 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
       }
       if (!is_two) {
         bswap(k, one_at);
-        if (!(ldl_mod(A[k]) > LDL_PIVOT_TOLERANCE * sc[od[k]])) {
+        if (!(ldl_mod(A[k]) > LDL_PIVOT_TOLERANCE * (one_at == k ? sk : sc[od[k]]))) {
           failed = k;
           break;
         }
@@ -469,7 +528,11 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
         const T d = A[k];
         const int64_t start = ldl_offset(m, k);
         for (int64_t r = k + threadIdx.x; r < m; r += blockDim.x) own[start + r - k] = r == k ? d : A[r] / d;
-        if (threadIdx.x == 0) pv[k] = PIV_ONE;
+        if (threadIdx.x == 0) {
+          pv[k] = PIV_ONE;
+          pk[k - c0] = PIV_ONE;
+          d1[k - c0] = d;
+        }
         __syncthreads();
         k += 1;
       } else {
@@ -497,6 +560,11 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
           own[q1] = d22;
           pv[k] = PIV_FIRST;
           pv[k + 1] = PIV_SECOND;
+          pk[k - c0] = PIV_FIRST;
+          pk[k + 1 - c0] = PIV_SECOND;
+          d1[k - c0] = d11;
+          d2[k - c0] = d21;
+          d1[k + 1 - c0] = d22;
         }
         twos += 1;
         __syncthreads();
@@ -512,11 +580,7 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
       }
       break;
     }
-    for (int64_t cb = c1; cb < w; cb += LDL_YC)
-      ldl_update(own, m, own, m, c0, (int)(c1 - c0), pv + c0, c1, m - c1, w - c1, nullptr, true, c1, cb,
-                 cb + LDL_YC < w ? cb + LDL_YC : w, cb, m);
-    __syncthreads();
-    c0 = c1;
+    c0 = c1;  // (one panel: w <= LDL_PANEL)
   }
   if (threadIdx.x == 0) {
     if (!ONE) {
@@ -568,8 +632,11 @@ __global__ __launch_bounds__(256) void k_ldlt_trailing(const LdlTile* __restrict
   if (state[4 * tl.j + 2] >= 0 || c1 >= J.w || c1 <= c0 || tl.e <= c1) return;
   const int64_t m = J.m, w = J.w;
   T* own = val + J.voff;
-  ldl_update(own, m, own, m, c0, (int)(c1 - c0), piv + J.first + c0, c1, m - c1, w - c1, nullptr, true, c1,
-             tl.b > c1 ? tl.b : c1, tl.e, tl.rb, tl.re);
+  // target (r, c) = c1 + (i, c): the tile's columns and rows past the panel
+  const int64_t ca = (tl.b > c1 ? tl.b : c1) - c1, cz = (tl.e < w ? tl.e : w) - c1;
+  const int64_t ia = (tl.rb > c1 ? tl.rb : c1) - c1, iz = (tl.re < m ? tl.re : m) - c1;
+  if (ca >= cz || ia >= iz) return;  // uniform
+  ldl_update(own, m, own, m, c0, (int)(c1 - c0), piv + J.first + c0, c1, (const int32_t*)nullptr, c1, ca, cz, ia, iz);
 }
 
 // D's blocks for the inertia: out[2 c] = D(c, c), out[2 c + 1] = D(c + 1, c) at the first column
@@ -605,31 +672,56 @@ __global__ __launch_bounds__(256) void k_ldlt_fwd_gather(const LdlTile* __restri
                                                          const T* __restrict__ val, const T* __restrict__ z,
                                                          T* __restrict__ x) {
 #pragma clang fp contract(off)
+  constexpr int NU = 128;  // updates whose ranges are found together (as k_ldlt_assemble's)
+  constexpr int QB = sizeof(T) == 8 ? 16 : 8;  // columns in flight at a time
+  __shared__ int range[NU][2];
   const LdlTile tl = tiles[blockIdx.x];
   const LdlSupernode J = S[tl.j];
-  for (int64_t u = J.upd0; u < J.upd1; ++u) {
-    const LdlUpdate up = U[u];
-    const LdlSupernode K = S[up.k];
-    const int32_t* rl = rel + up.rel;  // rl[i]: the column of J that row p1 + i of K lands on
-    const int64_t cnt = up.p2 - up.p1;
-    int64_t ia = 0, iz = cnt, hi = cnt;
-    while (ia < hi) { const int64_t mid = (ia + hi) / 2; if (rl[mid] < tl.b) ia = mid + 1; else hi = mid; }
-    hi = cnt;
-    iz = ia;
-    while (iz < hi) { const int64_t mid = (iz + hi) / 2; if (rl[mid] < tl.e) iz = mid + 1; else hi = mid; }
-    const T* lk = val + K.voff;
-    const T* zk = z + K.first;
-    for (int64_t i = ia + threadIdx.x; i < iz; i += blockDim.x) {
-      T* xi = x + J.first + rl[i];
-      T v = *xi;
-      int64_t at = up.p1 + i;  // L_k(p1 + i, 0); column q + 1's entry lies K.m - q - 1 on
-      for (int64_t q = 0; q < K.w; ++q) {
-        v -= lk[at] * zk[q];
-        at += K.m - q - 1;
+  for (int64_t u0 = J.upd0; u0 < J.upd1; u0 += NU) {
+    __syncthreads();
+    {
+      const int t = threadIdx.x >> 1, which = threadIdx.x & 1;
+      int at = 0;
+      if (u0 + t < J.upd1) {
+        const LdlUpdate up = U[u0 + t];
+        at = ldl_first_at_least(rel + up.rel, up.p2 - up.p1, which == 0 ? tl.b : tl.e);
       }
-      *xi = v;
+      range[t][which] = at;
     }
     __syncthreads();
+    for (int t = 0; t < NU; ++t) {
+      const int ia = range[t][0], iz = range[t][1];
+      if (ia >= iz) continue;
+      const LdlUpdate up = U[u0 + t];
+      const LdlSupernode K = S[up.k];
+      const int32_t* rl = rel + up.rel;  // rl[i]: the column of J that row p1 + i of K lands on
+      const T* lk = val + K.voff;
+      const T* zk = z + K.first;
+      for (int i = ia + (int)threadIdx.x; i < iz; i += blockDim.x) {
+        T* xi = x + J.first + rl[i];
+        T v = *xi;
+        int64_t at = up.p1 + i;  // L_k(p1 + i, 0); column q + 1's entry lies K.m - q - 1 on
+        // whole batches with no test inside (a test would move each load behind it)
+        auto batch = [&](int q0, auto nb) {
+          constexpr int NB_ = decltype(nb)::value;
+          T l[NB_], zq[NB_];
+#pragma unroll
+          for (int j = 0; j < NB_; ++j) {
+            l[j] = lk[at];
+            zq[j] = zk[q0 + j];
+            at += K.m - (q0 + j) - 1;
+          }
+#pragma unroll
+          for (int j = 0; j < NB_; ++j) v -= l[j] * zq[j];
+        };
+        int q0 = 0;
+        for (; q0 + QB <= K.w; q0 += QB) batch(q0, std::integral_constant<int, QB>{});
+        for (; q0 + 3 <= K.w; q0 += 3) batch(q0, std::integral_constant<int, 3>{});
+        for (; q0 < K.w; ++q0) batch(q0, std::integral_constant<int, 1>{});
+        *xi = v;
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -691,115 +783,200 @@ __device__ __forceinline__ void ldl_bwd_col(const int8_t* pv, int64_t c, int64_t
 }
 
 // sum - b[0] - b[1] - ... - b[cnt - 1] in that order, the next 16 operands read from LDS while the
-// current 16 are used; b is 16-byte aligned and readable 16 entries past cnt.
+// current 16 are used (two sets of registers in turn); b is 16-byte aligned and readable 32 entries
+// past cnt. About 14 cycles a subtraction over a whole backward pass: the dependence bounds it.
 __device__ __forceinline__ double ldl_chain(double sum, const double* b, int cnt) {
 #pragma clang fp contract(off)
-  const int nb = cnt / 16;
+  const int nb = cnt / 32;
   const double2* p2 = reinterpret_cast<const double2*>(b);
-  double2 cur[8], nxt[8];
+  double2 e[8], o[8];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) cur[u] = p2[u];
-  for (int bt = 0; bt < nb; ++bt) {
+  for (int u = 0; u < 8; ++u) e[u] = p2[u];
+  for (int bt = 0; bt < nb; ++bt, p2 += 16) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) nxt[u] = p2[(bt + 1) * 8 + u];
+    for (int u = 0; u < 8; ++u) o[u] = p2[8 + u];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      sum -= cur[u].x;
-      sum -= cur[u].y;
+      sum -= e[u].x;
+      sum -= e[u].y;
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) cur[u] = nxt[u];
+    for (int u = 0; u < 8; ++u) e[u] = p2[16 + u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      sum -= o[u].x;
+      sum -= o[u].y;
+    }
   }
-  for (int r = nb * 16; r < cnt; ++r) sum -= b[r];
+  // the last 0 .. 31: operands past cnt as zeros (x - 0 is x)
+  const int rem = cnt - nb * 32;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) o[u] = p2[8 + u];
+  if (rem > 0)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      sum -= 2 * u < rem ? e[u].x : 0.0;
+      sum -= 2 * u + 1 < rem ? e[u].y : 0.0;
+    }
+  if (rem > 16)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      sum -= 16 + 2 * u < rem ? o[u].x : 0.0;
+      sum -= 16 + 2 * u + 1 < rem ? o[u].y : 0.0;
+    }
   return sum;
 }
 
 // The complex chain: sum - b[0] - ... - b[cnt - 1] by parts, one element per 16-byte read.
 __device__ __forceinline__ zd ldl_chain(zd sum, const zd* b, int cnt) {
 #pragma clang fp contract(off)
-  const int nb = cnt / 8;
+  const int nb = cnt / 16;
   const double2* p2 = reinterpret_cast<const double2*>(b);
-  double2 cur[8], nxt[8];
+  double2 e[8], o[8];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) cur[u] = p2[u];
-  for (int bt = 0; bt < nb; ++bt) {
+  for (int u = 0; u < 8; ++u) e[u] = p2[u];
+  for (int bt = 0; bt < nb; ++bt, p2 += 16) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) nxt[u] = p2[(bt + 1) * 8 + u];
+    for (int u = 0; u < 8; ++u) o[u] = p2[8 + u];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      sum.re -= cur[u].x;
-      sum.im -= cur[u].y;
+      sum.re -= e[u].x;
+      sum.im -= e[u].y;
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) cur[u] = nxt[u];
+    for (int u = 0; u < 8; ++u) e[u] = p2[16 + u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      sum.re -= o[u].x;
+      sum.im -= o[u].y;
+    }
   }
-  for (int r = nb * 8; r < cnt; ++r) sum = sum - b[r];
+  const int rem = cnt - nb * 16;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) o[u] = p2[8 + u];
+  if (rem > 0)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      sum.re -= u < rem ? e[u].x : 0.0;
+      sum.im -= u < rem ? e[u].y : 0.0;
+    }
+  if (rem > 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      sum.re -= 8 + u < rem ? o[u].x : 0.0;
+      sum.im -= 8 + u < rem ? o[u].y : 0.0;
+    }
   return sum;
 }
 
-constexpr int LDL_BW_CAP = 3840;  // products of one column held in LDS (two such buffers)
+constexpr int LDL_BW_CAP = 3840;    // products of one column held in LDS (two such buffers)
+constexpr int LDL_BW_SMALL = 1024;  // the same for levels whose supernodes have no more rows
 
 // The backward pass (cholesky.rs:982-1030) for the supernodes of one level (sn[blockIdx.x]),
 // levels from the root down: a supernode's unknowns are its own and its sums read only its
 // ancestors' (final) unknowns, so the supernodes of a level are independent. Each sum runs in
-// the reference's order on one lane. With m <= cap (<= LDL_BW_CAP), waves 1.. stage the next column's
+// the reference's order on one lane. With m <= cap (<= CAP), waves 1.. stage the next column's
 // products while lane 0 runs the current column's sum: the one product that needs the unknown
 // being finished (its row is the current column's q) is left to lane 0, which forms it first.
 // Larger supernodes stage each column in chunks before its sum.
-template <typename T>
+// Bound by lane 0's chain of dependent subtractions: on a tet10 block of 8 cells a side (13 872
+// unknowns, the widest chains of the levels 2.54 million subtractions together) the pass takes 15 ms;
+// 24 ms with the levels by height (3.99 million). What the staging reads beside the column itself
+// (the unknowns of all m rows, the pivot kinds) is taken to LDS once, and PRE entries a thread of the
+// column after the staged one are in flight, so that short columns are not bound by two or three
+// loads one behind another instead (2 % of the pass there).
+// CAP = LDL_BW_SMALL leaves room for several workgroups a CU where a level has many small supernodes.
+template <typename T, int CAP>
 __global__ __launch_bounds__(256) void k_ldlt_solve_bwd(const int64_t* __restrict__ sn, const LdlSupernode* __restrict__ S,
                                                        const int64_t* __restrict__ rows_all, const T* __restrict__ val,
                                                        const int8_t* __restrict__ piv, const int32_t* __restrict__ order,
                                                        T* __restrict__ x, T* __restrict__ ywork, int cap) {
 #pragma clang fp contract(off)
+  constexpr int PL = CAP + 32;                                          // one buffer of products
+  constexpr int ROOM = (160 * 1024 - 256 - CAP) / (int)sizeof(T) - 2 * PL;  // entries of LDS left for the unknowns
+  constexpr int VC = ROOM < CAP ? ROOM : CAP;
+  constexpr int ST = 192;       // staging threads
+  constexpr int PRE = 6;        // entries a thread holds of a column (6 x 192 > LDL_BW_SMALL)
   const LdlSupernode K = S[sn[blockIdx.x]];
-  const int64_t m = K.m, w = K.w;
+  const int m = K.m, w = K.w;
   const T* t = val + K.voff;
   const int8_t* pv = piv + K.first;
   const int32_t* od = order + K.first;
   const int64_t* rows = rows_all + K.rows;
   T* own = x + K.first;
   T* y = ywork + K.first;
-  if (cap < 16 || cap > LDL_BW_CAP) cap = LDL_BW_CAP;
-  __shared__ __align__(16) T P[2][LDL_BW_CAP + 16];
+  if (cap < 16 || cap > CAP) cap = CAP;
+  __shared__ __align__(16) T P[2][PL];
+  __shared__ T V[VC];
+  __shared__ int8_t pvs[CAP];
   __shared__ T Lr[2];      // L(late row, q) of the staged column
-  __shared__ int64_t late[2];   // position of its late product, or -1
+  __shared__ int late[2];  // position of its late product, or -1
   __shared__ T acc;
-  for (int64_t c = threadIdx.x; c < w; c += blockDim.x) y[c] = own[c];
-  __syncthreads();
-  if (m <= cap && blockDim.x > 64) {
-    {
+  // at(r): the unknown of row r (r >= w: an ancestor's), put(q, v): unknown q is v
+  auto staged = [&](auto at, auto put) {
+    for (int c = threadIdx.x; c < w; c += blockDim.x) pvs[c] = pv[c];
+    __syncthreads();
+    const int tid = (int)threadIdx.x - 64;  // staging thread
+    T pre[PRE];
+    // the first PRE entries a thread has of pivot position c's column
+    auto fetch = [&](int c) {
       int64_t q, end;
-      ldl_bwd_col(pv, w - 1, q, end);  // end = w: every product reads an ancestor's unknown
+      ldl_bwd_col(pvs, c, q, end);
       const T* col = t + ldl_offset(m, q) - q;
-      for (int64_t r = end + threadIdx.x; r < m; r += blockDim.x) P[0][r - end] = col[r] * (r < w ? y[r] : x[rows[r]]);
-      if (threadIdx.x == 0) late[0] = -1;
+#pragma unroll
+      for (int j = 0; j < PRE; ++j) pre[j] = col[min((int)end + tid + ST * j, m - 1)];
+    };
+    // its products, but for row `skip`, into P[b]
+    auto stage = [&](int c, int b, int skip) {
+      int64_t q64, end64;
+      ldl_bwd_col(pvs, c, q64, end64);
+      const int end = (int)end64;
+      const T* col = t + ldl_offset(m, q64) - q64;
+#pragma unroll
+      for (int j = 0; j < PRE; ++j) {
+        const int r = end + tid + ST * j;
+        if (r < m && r != skip) P[b][r - end] = pre[j] * at(r);
+        if (r < m && r == skip) Lr[b] = pre[j];
+      }
+      for (int r = end + tid + ST * PRE; r < m; r += ST) {
+        const T l = col[r];
+        if (r != skip) P[b][r - end] = l * at(r);
+        else Lr[b] = l;
+      }
+      if (tid == 0) late[b] = skip >= end ? skip - end : -1;
+    };
+    if (tid >= 0) {
+      fetch(w - 1);
+      stage(w - 1, 0, -1);  // every product reads an ancestor's unknown
+      if (w > 1) fetch(w - 2);
     }
     __syncthreads();
-    for (int64_t c = w - 1; c >= 0; --c) {
-      const int cur = (int)((w - 1 - c) & 1), nx = cur ^ 1;
+    T last = T{};  // lane 0: the unknown finished last
+    for (int c = w - 1; c >= 0; --c) {
+      const int cur = (w - 1 - c) & 1;
       int64_t q, end;
-      ldl_bwd_col(pv, c, q, end);
+      ldl_bwd_col(pvs, c, q, end);
       if (threadIdx.x == 0) {
-        if (late[cur] >= 0) P[cur][late[cur]] = Lr[cur] * y[end + late[cur]];
-        y[q] = ldl_chain(y[q], P[cur], (int)(m - end));
-      } else if (threadIdx.x >= 64 && c > 0) {
-        int64_t qn, en;
-        ldl_bwd_col(pv, c - 1, qn, en);
-        const T* col = t + ldl_offset(m, qn) - qn;
-        for (int64_t r = en + (threadIdx.x - 64); r < m; r += blockDim.x - 64)
-          if (r != q) P[nx][r - en] = col[r] * (r < w ? y[r] : x[rows[r]]);
-        if (threadIdx.x == 64) {
-          if (q >= en) {
-            late[nx] = q - en;
-            Lr[nx] = col[q];
-          } else {
-            late[nx] = -1;
-          }
-        }
+        if (late[cur] >= 0) P[cur][late[cur]] = Lr[cur] * last;
+        last = ldl_chain(at((int)q), P[cur], m - (int)end);
+        put((int)q, last);
+      } else if (tid >= 0 && c > 0) {
+        stage(c - 1, cur ^ 1, (int)q);
+        if (c > 1) fetch(c - 2);
       }
       __syncthreads();
     }
+  };
+  if (m <= cap && m <= VC) {
+    for (int r = threadIdx.x; r < m; r += blockDim.x) V[r] = r < w ? own[r] : x[rows[r]];
+    staged([&](int r) { return V[r]; }, [&](int q, T v) { V[q] = v; });
+    for (int c = threadIdx.x; c < w; c += blockDim.x) own[od[c]] = V[c];
+    return;
+  }
+  for (int c = threadIdx.x; c < w; c += blockDim.x) y[c] = own[c];
+  __syncthreads();
+  if (m <= cap) {
+    staged([&](int r) { return r < w ? y[r] : x[rows[r]]; }, [&](int q, T v) { y[q] = v; });
   } else {
     for (int64_t c = w - 1; c >= 0; --c) {
       int64_t q, end;
@@ -817,7 +994,7 @@ __global__ __launch_bounds__(256) void k_ldlt_solve_bwd(const int64_t* __restric
       __syncthreads();
     }
   }
-  for (int64_t c = threadIdx.x; c < w; c += blockDim.x) own[od[c]] = y[c];
+  for (int c = threadIdx.x; c < w; c += blockDim.x) own[od[c]] = y[c];
 }
 
 }  // namespace fc
