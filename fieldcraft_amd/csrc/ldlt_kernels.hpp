@@ -487,10 +487,11 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
         int step = 0;
         for (;;) {
           current(c0, k, r, B);
+          // (B(r) before the barrier in `largest`: a wave ahead may interchange B's entries after it)
+          const double arr = ldl_mod(B[r]);
           int64_t s_at;
           double omega_r;
           largest(B, k, w, r, &s_at, &omega_r);
-          const double arr = ldl_mod(B[r]);
           if (!isfinite(arr) || !isfinite(omega_r)) {
             failed = k;
             break;
