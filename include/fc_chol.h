@@ -57,9 +57,8 @@ typedef enum {
   FC_FP64 = 0,  /* the plain method: every step in FP64 on the FP64 matrix cores           */
   FC_MIXED = 1, /* Schur updates in BF16 (power-of-two scaled, FP32 accumulation), the rows
                    below a panel (TRSM) on the FP32 matrix cores, diagonal blocks factored
-                   and inverted in FP32 arithmetic (a block with a pivot below 1e-3 |A_jj|
-                   is factored again in FP64 arithmetic, where the reference's pivot test
-                   decides); the factor is stored in FP32; solutions are refined in FP64   */
+                   and inverted in FP64 arithmetic; the factor is stored in FP32; solutions
+                   are refined in FP64                                                     */
   FC_FP32 = 2   /* every step in FP32 (diagonal blocks as FC_MIXED's), factor stored in FP32 */
 } fc_precision;
 
