@@ -31,8 +31,8 @@
 // a block backward, 6 us forward (FP64, the 36^3 cube's root of 49 blocks), and below them the
 // levels' launches. Measured against a launch a block on the vector units, with a launch of one workgroup
 // a front to gather and one to start each level: 8 right-hand sides of the 20 x 23 x 17 hex8 block
-// 2.78 -> 0.85 ms; a refined solve of 16 vectors on the mixed factor of the 13^3 tet10 block 25.0 ->
-// 6.2 ms; one right-hand side of the 36^3 cube (one launch a level before, too) 3.60 -> 2.46 ms.
+// 2.78 -> 0.76 ms; a refined solve of 16 vectors on the mixed factor of the 13^3 tet10 block 25.0 ->
+// 5.6 ms; one right-hand side of the 36^3 cube (one launch a level before, too) 3.60 -> 2.22 ms.
 #pragma once
 
 #include <type_traits>
