@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256, 2) void k_small_fronts(const Item* __restrict_
 #pragma unroll
     for (int k = 0; k < NBK; ++k) {
       if (k >= nb) break;
-      substitute_block<double, sizeof(T) == 8>(
+      substitute_block<double, sizeof(T) == 8, false>(
           x, k, [&](int j, int s) { return S[16 * k + r][16 * j + 4 * s + g]; },
           [&](int s) { return X[k][4 * s + g][r]; },
           [&](int s) {
