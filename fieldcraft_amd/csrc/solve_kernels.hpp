@@ -122,15 +122,16 @@ __device__ __forceinline__ void to_lds(double (*V)[SRHS * NG], const v4d (&val)[
 }
 
 // Four consecutive entries of T at byte offset lane + off of a resource: two (FP64) or one 16-byte
-// loads, or where `part` is set one load an entry, those from `valid` on reading 0.
-template <typename T>
-__device__ __forceinline__ void load4(double (&a)[4], __amdgpu_buffer_rsrc_t rs, uint32_t lane, uint32_t off, bool part,
+// loads, or where `part` is set one load an entry, those from `valid` on reading 0. As they lie in
+// memory, or converted to V.
+template <typename T, typename V>
+__device__ __forceinline__ void load4(V (&a)[4], __amdgpu_buffer_rsrc_t rs, uint32_t lane, uint32_t off, bool part,
                                       int valid) {
+  typedef unsigned int u32x4 __attribute__((__vector_size__(16)));
   if (part) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) a[s] = (double)buf_load<T>(rs, s < valid ? lane + s * (uint32_t)sizeof(T) : 0x80000000u, off);
+    for (int s = 0; s < 4; ++s) a[s] = (V)buf_load<T>(rs, s < valid ? lane + s * (uint32_t)sizeof(T) : 0x80000000u, off);
   } else if constexpr (sizeof(T) == 8) {
-    typedef unsigned int u32x4 __attribute__((__vector_size__(16)));
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, lane + 16 * h, off, 0);
@@ -138,12 +139,11 @@ __device__ __forceinline__ void load4(double (&a)[4], __amdgpu_buffer_rsrc_t rs,
       a[2 * h + 1] = __builtin_bit_cast(double, (uint64_t)w[2] | (uint64_t)w[3] << 32);
     }
   } else {
-    typedef unsigned int u32x4 __attribute__((__vector_size__(16)));
     const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, lane, off, 0);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const unsigned e = w[s];  // (a bit cast of the vector's element itself reads element 0)
-      a[s] = (double)__builtin_bit_cast(float, e);
+      a[s] = (V)__builtin_bit_cast(float, e);
     }
   }
 }
@@ -332,18 +332,30 @@ __device__ __forceinline__ void below_products(v4d (&acc)[CB][NG], const FrontDe
   for (int cb = 0; cb < CB; ++cb)
     lo[cb] = (uint32_t)(min(j0 + 16 * cb + r, F.w - 1) - j0) * F.ld * sizeof(T) + 4 * q * (uint32_t)sizeof(T);
   // BT steps of 16 rows at a time, every load of theirs in flight together; the next ones' column
-  // numbers are read with them
+  // numbers are read with them. In FP32 a lane's four by one load: an entry costs half the bytes there, so the
+  // instructions beside it count (a load each in FP64: by one load its 8-side solve took 2 % longer).
+  const auto ri = raw_rsrc(below);
   auto index = [&](int it, int (&ix)[BT][4]) {
 #pragma unroll
-    for (int t = 0; t < BT; ++t)
+    for (int t = 0; t < BT; ++t) {
+      const int b = 16 * (it + t * step);
+      if constexpr (sizeof(T) == 4) {
+        float e[4];
+        load4<float>(e, ri, 16 * q, (uint32_t)b * 4, b + 16 > mu, mu - b - 4 * q);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) ix[t][s] = below[min(16 * (it + t * step) + 4 * q + s, mu - 1)];
+        for (int s = 0; s < 4; ++s) ix[t][s] = __builtin_bit_cast(int, e[s]);
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) ix[t][s] = below[min(b + 4 * q + s, mu - 1)];
+      }
+    }
   };
   if (16 * it0 >= mu) return;
   int ix[BT][4];
   index(it0, ix);
   for (int it = it0; 16 * it < mu; it += BT * step) {
-    double a[BT][CB][4], x[BT][NG][4];
+    T a[BT][CB][4];
+    double x[BT][NG][4];
 #pragma unroll
     for (int t = 0; t < BT; ++t) {
       const int b = 16 * (it + t * step);
@@ -366,12 +378,17 @@ __device__ __forceinline__ void below_products(v4d (&acc)[CB][NG], const FrontDe
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-            for (int g = 0; g < NG; ++g) acc[cb][g] = Mma<double>::step(a[t][cb][s], x[t][g][s], acc[cb][g]);
+            for (int g = 0; g < NG; ++g) acc[cb][g] = Mma<double>::step((double)a[t][cb][s], x[t][g][s], acc[cb][g]);
   }
 }
 
 // Backward, item (f, a = j0): z_j = y_j - L21(:, j)^T x_below for the columns j0 .. j0 + 16 CB - 1, in
-// place in y. The eight waves share the rows; their sums are added in order.
+// place in y. The eight waves share the rows; their sums are added in order. Bound: memory, through as
+// many loads in flight as registers allow. FP32 holds its operands unconverted, and where a step loads two
+// column blocks takes two steps at a time, not four: 86 registers leave a CU two workgroups. With
+// four steps, converted operands (160 registers, one workgroup) and a load for each column number the
+// launches of one side on the 80^3 hex8 factor took 5.4 ms, now 4.2; FP64 keeps four steps (two: 2 % slower
+// with 8 sides).
 template <typename T, int NG, int CB>
 __global__ __launch_bounds__(STHREADS) void k_bwd_below(const Item* __restrict__ items,
                                                         const FrontDev* __restrict__ fronts, const T* __restrict__ L,
@@ -388,7 +405,7 @@ __global__ __launch_bounds__(STHREADS) void k_bwd_below(const Item* __restrict__
   for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
     for (int g = 0; g < NG; ++g) acc[cb][g] = v4d{0, 0, 0, 0};
-  below_products<T, NG, CB, (NG * CB > 2 ? 2 : 4)>(acc, F, L, rows, xp, sd, it.a, wave, 8, lane);
+  below_products<T, NG, CB, (NG * CB > 2 || (sizeof(T) == 4 && CB > 1) ? 2 : 4)>(acc, F, L, rows, xp, sd, it.a, wave, 8, lane);
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
 #pragma unroll
