@@ -858,6 +858,7 @@ struct fc_factor {
   struct SolveGraph {                  // opts.use_graph bit 1: a captured solve
     int nr;
     void *xp, *yp, *u, *err;
+    int64_t limit;  // a kernel argument too
     hipGraph_t g;
     hipGraphExec_t exec;
   };
@@ -1272,13 +1273,6 @@ int factor_host(fc_factor* F, const double* upper_val, uint64_t nnz, fc_error* e
   }
 }
 
-// A solve pass's device work: x and y (n x nr, the right-hand sides of an equation side by side), the
-// fronts' contributions, and the error word of the chains (set when a wait gave up).
-struct SolveWork {
-  double *xp, *yp, *u;
-  int32_t* err;
-};
-
 // The polls a chained solve's wait may take before it gives up (FC_SOLVE_SPIN_LIMIT; negative:
 // every wait gives up at once, a test's way to reach the failure path).
 int64_t solve_spin_limit() {
@@ -1286,12 +1280,19 @@ int64_t solve_spin_limit() {
   return (int64_t)1 << 22;
 }
 
+// A solve pass's device work: x and y (n x nr, the right-hand sides of an equation side by side), the
+// fronts' contributions, the error word of the chains (set when a wait gave up) and their waits' limit.
+struct SolveWork {
+  double *xp, *yp, *u;
+  int32_t* err;
+  int64_t limit = solve_spin_limit();
+};
+
 template <typename T, int NG>
 void run_solve_ng(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st) {
   DevicePlan& P = *F->plan;
   const T* L = (const T*)F->L;
   const T* Inv = (const T*)F->inv.p;
-  const int64_t limit = solve_spin_limit();
   const int groups = (nr + fc::SRHS * NG - 1) / (fc::SRHS * NG);
   auto run = [&](const fc::Launch& l) {
     const fc::Item* it = P.sitems + l.item0;
@@ -1299,7 +1300,7 @@ void run_solve_ng(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st
     switch (l.kind) {
       case S_FWD:
         fc::k_fwd<T, NG><<<g, b, 0, st>>>(it, P.fronts, P.gptr, P.gsrc, L, Inv, w.xp, w.yp, w.u, P.uoff, nr, l.count,
-                                          w.err, limit);
+                                          w.err, w.limit);
         break;
       case S_FWD_ONE:
         fc::k_fwd_one<T, NG><<<g, b1, 0, st>>>(it, P.fronts, P.gptr, P.gsrc, L, Inv, w.xp, w.yp, w.u, P.uoff, nr, l.count);
@@ -1309,7 +1310,7 @@ void run_solve_ng(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st
         else fc::k_bwd_below<T, NG, 2><<<g, b, 0, st>>>(it, P.fronts, L, P.rows, w.xp, w.yp, nr, l.count);
         break;
       case S_BWD:
-        fc::k_bwd<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, P.rows, w.yp, w.xp, nr, l.count, w.err, limit);
+        fc::k_bwd<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, P.rows, w.yp, w.xp, nr, l.count, w.err, w.limit);
         break;
       case S_BWD_ONE:
         fc::k_bwd_one<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, P.rows, w.yp, w.xp, nr, l.count);
@@ -1328,7 +1329,7 @@ void run_solve(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st) {
 }
 
 // The solve's launches for nr right-hand sides in w, replayed from a hipGraph when
-// opts.use_graph asks for it (bit 1): captured on first use for each (nr, workspaces).
+// opts.use_graph asks for it (bit 1): captured on first use for each (nr, workspaces, limit).
 void solve_launches(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st) {
   auto eager = [&]() {
     if (F->precision == FC_FP64) run_solve<double>(F, w, nr, st);
@@ -1336,11 +1337,11 @@ void solve_launches(const fc_factor* F, const SolveWork& w, int nr, hipStream_t 
   };
   if (!(F->opts.use_graph & 2)) return eager();
   for (const auto& sg : F->sgraphs)
-    if (sg.nr == nr && sg.xp == w.xp && sg.yp == w.yp && sg.u == w.u && sg.err == w.err) {
+    if (sg.nr == nr && sg.xp == w.xp && sg.yp == w.yp && sg.u == w.u && sg.err == w.err && sg.limit == w.limit) {
       HIP_CHECK(hipGraphLaunch(sg.exec, st));
       return;
     }
-  fc_factor::SolveGraph sg{nr, w.xp, w.yp, w.u, w.err, nullptr, nullptr};
+  fc_factor::SolveGraph sg{nr, w.xp, w.yp, w.u, w.err, w.limit, nullptr, nullptr};
   HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   try {
     eager();

@@ -230,3 +230,24 @@ def test_reduced_precision_falls_back_to_fp64_storage(gpu, monkeypatch, precisio
     g.refactor(up.val)
     assert g.precision_used() == "fp64"
     check_fp64(g, ref, up, b, xr)
+
+
+@pytest.mark.parametrize("graph", [0, 2])
+@pytest.mark.parametrize("nrhs", [1, 17])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_a_solves_wait_that_gives_up_is_an_error(gpu, cube16, monkeypatch, precision, nrhs, graph):
+    """A negative FC_SOLVE_SPIN_LIMIT makes every wait of the block chains give up at once (the root is
+    870 columns, seven blocks): the solve reports a device error, whether its launches are issued or
+    replayed from a graph captured before, and the next one with the limit lifted is the bits of one
+    before it."""
+    p, up, sym, e = cube16
+    f = CH.Factor(sym, up[2], precision=precision, use_graph=graph)
+    bs = [np.cos(0.01 * k) * p.rhs for k in range(nrhs)]
+    before = f.solve_many(bs)
+    monkeypatch.setenv("FC_SOLVE_SPIN_LIMIT", "-1")
+    for _ in range(2):
+        with pytest.raises(CH.DeviceError):
+            f.solve_many(bs)
+    monkeypatch.delenv("FC_SOLVE_SPIN_LIMIT")
+    for x, x0 in zip(f.solve_many(bs), before):
+        assert np.array_equal(x, x0)
