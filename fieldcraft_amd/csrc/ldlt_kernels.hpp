@@ -25,7 +25,10 @@ enum : int8_t { PIV_ONE = 0, PIV_FIRST = 1, PIV_SECOND = 2 };
 
 // The complex scalar of complex-symmetric LDL^T (ldlt.rs over Complex64, scalar.rs:115-131) with
 // num-complex 0.4's arithmetic: products (ac - bd, ad + bc), quotients by the squared norm, sums
-// by parts; the modulus hypot(re, im) for the pivot tests. Transposes, never conjugates.
+// by parts; the modulus hypot(re, im) for the pivot tests. Transposes, never conjugates. A 2 x 2 pivot is
+// settled between two computed values of one entry; where their moduli tie to a rounding, hypot's last
+// bit, in which libraries differ (glibc's is off the nearest double for 0.6 % of random arguments), can
+// settle it the other way: the factor is then another of the same search, not the reference's bits.
 struct zd {
   double re, im;
 };

@@ -87,3 +87,36 @@ def test_singular_complex_matrix_and_argument_errors(gpu):
     err = CH._Error()
     x = np.zeros(a[0])
     assert CH.lib().fc_ldlt_solve(f._h, x, a[0], CH.C.byref(err)) != 0  # a real solve of a complex factor
+
+
+@pytest.mark.parametrize("wa, rows, wd, chunk", [(90, 920, 960, None), (150, 1080, 1200, None), (150, 1080, 1200, "512"),
+                                                 (60, 2200, 2300, None)])
+@pytest.mark.parametrize("values", ["real", "dominant"])
+def test_tall_complex_supernodes_match_the_oracle_bit_for_bit(gpu, monkeypatch, wa, rows, wd, chunk, values):
+    """A block of wa columns with `rows` rows below it in a dense block of wd columns: supernodes of more
+    rows than the backward pass's small form takes (1 024), than the unknowns its LDS has room for beside
+    two columns of products (2 240 complex ones) and, with FC_LDLT_SOLVE_ROWS, than it stages of a
+    column at a time. A 2 x 2 pivot is chosen between two computed values of one entry, a tie to a
+    rounding in which the last bit of hypot decides, and libraries differ in it. The values are therefore
+    real, where the modulus is exact and a third of the pivots are 2 x 2, or complex with a diagonal that
+    every search stops at; the right-hand sides are complex."""
+    n = wa + wd
+    g = np.random.default_rng(n).uniform(-1.0, 1.0, (2, n, n))
+    d = g[0] + (0j if values == "real" else 1j * g[1])
+    d = (d + d.T) / 2.0
+    if values == "dominant":
+        d += 4.0 * np.sqrt(n) * np.diag(np.exp(1j * np.arange(n)))
+    d[:wa, wa + rows:] = 0.0
+    d[wa + rows:, :wa] = 0.0
+    ptr = np.concatenate([[0], np.cumsum((d != 0).sum(axis=1))])
+    a = (n, ptr, np.nonzero(d)[1], d[d != 0])
+    print(f"supernodes of {wa + rows} and {wd} rows, {values}", flush=True)
+    f, o = device(a), O.ZLdltFactor(n, *upper(a))
+    e = f.symbolic.export()
+    assert np.array_equal(np.diff(e["rptr"]), [wa + rows, wd]) and np.array_equal(np.diff(e["first"]), [wa, wd])
+    assert f.two_by_two() == o.two_by_two() and (o.two_by_two() > 0) == (values == "real")
+    assert np.array_equal(bits(f.values()), bits(o.values()))
+    if chunk:
+        monkeypatch.setenv("FC_LDLT_SOLVE_ROWS", chunk)
+    b = cmul(a, sample_solution(n))
+    assert np.array_equal(bits(f.solve(b)), bits(o.solve(b)))
