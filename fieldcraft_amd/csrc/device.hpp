@@ -14,14 +14,12 @@ namespace fc {
 struct FrontDev {
   int64_t lpos;
   int64_t upos;
-  int64_t rel_off;   // relative map of the rows below into the parent front
   int64_t rows_off;  // front rows (postorder column numbers) in the rows array
   int64_t inv0;      // inverses of the diagonal blocks: panel at c0 at inv0 + (c0 / NB) NB^2, ld = its width
   int64_t bpos;      // mixed form: BF16 copies of the L part, (i, j) at bpos + ((j / 32) ld + i) 32 + j % 32
   int32_t ld, w, m, col0;
-  int32_t parent, kid0, kid1, level;  // children are kids[kid0..kid1)
 };
-static_assert(sizeof(FrontDev) == 80, "FrontDev layout");
+static_assert(sizeof(FrontDev) == 56, "FrontDev layout");
 
 // Strided runs of loads (and stores) through a buffer resource: the lane's part of the address
 // is one VGPR offset and each access's part a scalar, so a run of independent accesses needs no

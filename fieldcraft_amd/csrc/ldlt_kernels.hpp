@@ -73,23 +73,6 @@ struct LdlUpdate {
 __device__ __forceinline__ int64_t ldl_offset(int64_t m, int64_t c) { return c * m - c * (c > 0 ? c - 1 : 0) / 2; }
 #define LDL_AT(t, m, r, c) ((t)[ldl_offset((m), (c)) + (r) - (c)])
 
-// Entry k of times_d(row) (cholesky.rs:460-484) for the row `row(j)` of a trapezoid t (m rows)
-// over its columns k0..: a 1 x 1 pivot scales, a 2 x 2 pivot mixes the pair with D's block.
-template <typename T, typename Row>
-__device__ __forceinline__ T times_d_at(const Row& row, const T* t, int64_t m, int64_t k0,
-                                             const int8_t* piv, int k, int len) {
-#pragma clang fp contract(off)
-  if (piv[k] == PIV_FIRST) {
-    const T a = row(k), b = k + 1 < len ? row(k + 1) : T{};
-    return a * LDL_AT(t, m, k0 + k, k0 + k) + b * LDL_AT(t, m, k0 + k + 1, k0 + k);
-  }
-  if (piv[k] == PIV_SECOND && k > 0 && piv[k - 1] == PIV_FIRST) {
-    const T a = row(k - 1), b = row(k);
-    return a * LDL_AT(t, m, k0 + k, k0 + k - 1) + b * LDL_AT(t, m, k0 + k, k0 + k);
-  }
-  return row(k) * LDL_AT(t, m, k0 + k, k0 + k);
-}
-
 constexpr int LDL_YC = 16;   // target columns of one update window (and one tile)
 constexpr int LDL_KC = 128;  // source columns of Y staged in LDS at a time
 constexpr int LDL_PP = 8;    // pairs per thread per batch
@@ -304,7 +287,6 @@ __device__ __forceinline__ int ldl_wave_min(int v) {
 // column (or stays -1); two[s] the supernode's 2 x 2 pivots.
 template <typename T, bool ONE>
 __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restrict__ sn, const LdlSupernode* __restrict__ S,
-                                                        const LdlUpdate* __restrict__ U, const int32_t* __restrict__ rel,
                                                         const double* __restrict__ scale, T* __restrict__ val,
                                                         int8_t* __restrict__ piv, int32_t* __restrict__ order,
                                                         T* __restrict__ work, int64_t* __restrict__ fail,
@@ -316,8 +298,6 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
   T* own = val + J.voff;
   int8_t* pv = piv + J.first;
   int32_t* od = order + J.first;
-  (void)U;
-  (void)rel;
   int64_t* st = state + 4 * j;  // ONE: start and end of the last panel, failure, 2 x 2 pivots
   if (!ONE) {
     for (int64_t c = threadIdx.x; c < w; c += blockDim.x) {
@@ -348,7 +328,7 @@ __global__ __launch_bounds__(1024) void k_ldlt_supernode(const int64_t* __restri
   auto current = [&](int64_t c0, int64_t k, int64_t c, T* out) {
     const int n = (int)(k - c0);
     auto row = [&](int q) { return LDL_AT(own, m, c, c0 + q); };
-    if ((int)threadIdx.x < n) {  // times_d (cholesky.rs:460-484) of row c, as times_d_at
+    if ((int)threadIdx.x < n) {  // times_d (cholesky.rs:460-484) of row c: a 1 x 1 pivot scales, a 2 x 2 pivot mixes the pair
       const int q = threadIdx.x;
       const T a = row(q), lo = row(q > 0 ? q - 1 : 0), hi = row(q + 1 < n ? q + 1 : q);
       T y;

@@ -665,7 +665,6 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
 struct DeviceStruct {
   int device = -1;
   fc::FrontDev* fronts = nullptr;
-  int32_t* kids = nullptr;
   int32_t* rel = nullptr;
   int32_t* rows = nullptr;
   int64_t* a_pos = nullptr;
@@ -678,7 +677,7 @@ struct DeviceStruct {
     int cur = 0;
     (void)hipGetDevice(&cur);
     (void)hipSetDevice(device);
-    for (void* q : {(void*)fronts, (void*)kids, (void*)rel, (void*)rows, (void*)a_pos, (void*)diag_src, (void*)perm,
+    for (void* q : {(void*)fronts, (void*)rel, (void*)rows, (void*)a_pos, (void*)diag_src, (void*)perm,
                     (void*)gptr, (void*)gsrc})
       dfree(q);
     (void)hipSetDevice(cur);
@@ -692,7 +691,6 @@ struct DevicePlan {
   const Program* prog = nullptr;  // the program the items come from (held by its users)
   std::shared_ptr<DeviceStruct> st;
   fc::FrontDev* fronts = nullptr;
-  int32_t* kids = nullptr;
   int32_t* rel = nullptr;
   int32_t* rows = nullptr;
   int64_t* a_pos = nullptr;
@@ -766,7 +764,6 @@ struct fc_symbolic {
         fc::FrontDev& d = fd[f];
         d.lpos = S.f_lpos[f];
         d.upos = S.f_upos[f] < 0 ? 0 : S.f_upos[f];
-        d.rel_off = S.f_rel_off[f];
         d.rows_off = S.f_rptr[f];
         d.inv0 = pr->f_inv0[f];  // per-front layouts: the same in every program of the analysis
         d.bpos = pr->f_bpos[f];
@@ -774,15 +771,9 @@ struct fc_symbolic {
         d.w = (int32_t)S.f_w[f];
         d.m = (int32_t)S.f_m[f];
         d.col0 = (int32_t)S.f_col0[f];
-        d.parent = (int32_t)S.f_parent[f];
-        d.kid0 = (int32_t)S.f_kptr[f];
-        d.kid1 = (int32_t)S.f_kptr[f + 1];
-        d.level = (int32_t)S.f_level[f];
       }
-      std::vector<int32_t> kids(S.f_kids.begin(), S.f_kids.end());
       std::vector<int32_t> rows(S.f_rows.begin(), S.f_rows.end());
       ds->fronts = dupload(fd, st);
-      ds->kids = dupload(kids, st);
       ds->rel = dupload(S.rel, st);
       ds->rows = dupload(rows, st);
       ds->a_pos = dupload(S.a_pos, st);
@@ -812,7 +803,6 @@ struct fc_symbolic {
     p->prog = pr.get();
     p->st = ds;
     p->fronts = ds->fronts;
-    p->kids = ds->kids;
     p->rel = ds->rel;
     p->rows = ds->rows;
     p->a_pos = ds->a_pos;
@@ -2334,13 +2324,12 @@ int ldlt_numeric(const fc_symbolic* h, const T* upper_val, uint64_t nnz, int32_t
       const unsigned wlds = lds_for(P.lvl_ptr[l] + narrow, P.lvl_ptr[l + 1], &wrows);
       if (narrow > 0)
         fc::k_ldlt_supernode<T, false><<<(unsigned)narrow, narrow < 256 ? LDL_PANEL_THREADS : 256, nlds, stq>>>(
-            lsn, F->S, dU, drel, dscale, fval, F->piv, F->order, dwork, dfail, dtwo, dstate, nrows);
+            lsn, F->S, dscale, fval, F->piv, F->order, dwork, dfail, dtwo, dstate, nrows);
       if (wide > 0) {
         fc::k_ldlt_state_init<<<(unsigned)wide, 256, 0, stq>>>(lsn + narrow, F->S, F->piv, F->order, dfail, dtwo, dstate);
         for (i64 i = P.pan_ptr[l]; i < P.pan_ptr[l + 1]; ++i) {
-          fc::k_ldlt_supernode<T, true><<<(unsigned)wide, LDL_PANEL_THREADS, wlds, stq>>>(lsn + narrow, F->S, dU, drel, dscale, fval,
-                                                                         F->piv, F->order, dwork, dfail, dtwo, dstate,
-                                                                         wrows);
+          fc::k_ldlt_supernode<T, true><<<(unsigned)wide, LDL_PANEL_THREADS, wlds, stq>>>(
+              lsn + narrow, F->S, dscale, fval, F->piv, F->order, dwork, dfail, dtwo, dstate, wrows);
           const i64 pt = P.pan_tile_ptr[i + 1] - P.pan_tile_ptr[i];
           if (pt > 0)
             fc::k_ldlt_trailing<<<(unsigned)pt, 256, 0, stq>>>(dptiles + P.pan_tile_ptr[i], F->S, fval, F->piv, dstate);
