@@ -627,22 +627,21 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
   }
   for (i64 l = s.levels - 1; l >= 0; --l) {
     sort_level(l);
-    // the products with the rows below of all but the one-block fronts with few of them
-    auto fused = [&](i64 f) { return blocks(f) <= 1 && s.f_m[f] - s.f_w[f] <= fc::BELOW_FUSE; };
+    // the products with the rows below
     i64 i0 = (i64)p.sitems.size(), count = 0;
     for (i64 q = s.lvl_ptr[l]; q < s.lvl_ptr[l + 1]; ++q) {
       const i64 f = s.lvl_fronts[q];
-      if (s.f_m[f] > s.f_w[f] && !fused(f)) count += (s.f_w[f] + 15) / 16;
+      if (s.f_m[f] > s.f_w[f]) count += (s.f_w[f] + 15) / 16;
     }
     const i64 cb = count < SOLVE_FEW ? 1 : 2;
     for (i64 q = s.lvl_ptr[l]; q < s.lvl_ptr[l + 1]; ++q) {
       const i64 f = s.lvl_fronts[q];
-      if (s.f_m[f] > s.f_w[f] && !fused(f))
+      if (s.f_m[f] > s.f_w[f])
         for (i64 j = 0; j < s.f_w[f]; j += 16 * cb) sitem(f, j, 0);
     }
     sadd(p.sbwd, S_BELOW, l, i0, (int32_t)cb);
     i0 = (i64)p.sitems.size();
-    for (const i64 f : one) sitem(f, 0, fused(f));
+    for (const i64 f : one) sitem(f, 0, 0);
     sadd(p.sbwd, S_BWD_ONE, l, i0);
     // by distance from the front's last block, across the level's fronts: every chain starts in
     // the first workgroups, and a block's x is formed by an earlier workgroup than its users
@@ -651,7 +650,7 @@ Program build_program(const fc::Symbolic& s, const Schedule& sched) {
     for (const i64 f : wide) depth = std::max<i64>(depth, blocks(f));
     for (i64 k = 0; k < depth; ++k)
       for (const i64 f : wide)
-        if (k < blocks(f)) sitem(f, blocks(f) - 1 - k, fused(f));
+        if (k < blocks(f)) sitem(f, blocks(f) - 1 - k, 0);
     sadd(p.sbwd, S_BWD, l, i0);
   }
   p.uoff.assign(s.f_soff.begin(), s.f_soff.end());
@@ -1300,10 +1299,10 @@ void run_solve_ng(const fc_factor* F, const SolveWork& w, int nr, hipStream_t st
         else fc::k_bwd_below<T, NG, 2><<<g, b, 0, st>>>(it, P.fronts, L, P.rows, w.xp, w.yp, nr, l.count);
         break;
       case S_BWD:
-        fc::k_bwd<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, P.rows, w.yp, w.xp, nr, l.count, w.err, w.limit);
+        fc::k_bwd<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, w.yp, w.xp, nr, l.count, w.err, w.limit);
         break;
       case S_BWD_ONE:
-        fc::k_bwd_one<T, NG><<<g, b, 0, st>>>(it, P.fronts, L, Inv, P.rows, w.yp, w.xp, nr, l.count);
+        fc::k_bwd_one<T, NG><<<g, b, 0, st>>>(it, P.fronts, Inv, w.yp, w.xp, nr, l.count);
         break;
     }
   };

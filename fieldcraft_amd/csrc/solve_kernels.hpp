@@ -10,29 +10,33 @@
 //
 // A front is solved by blocks of SNB = 128 columns, its factorization's panels, whose diagonal
 // blocks' inverses the factorization keeps (column-major, ld = the block's width, zeros above
-// the diagonal). One launch a level and direction (plus, backward, one for the products of the
-// rows below): a front's workgroups each take 128 of its rows (forward) or columns (backward)
-// through its blocks in order, and the one that finishes the rows or columns of a block forms that
-// block's solution. A block's solution formed elsewhere is waited for value by value: the values
-// to come are marked PENDING, a signalling NaN that no arithmetic produces, before the launch;
-// the forming workgroup writes each with a device-coherent atomic store and a waiting thread
-// polls its own values until they are not PENDING (no fence: each value is its own signal). A
-// workgroup waits only on workgroups of its own front placed earlier in the launch, so the waits
-// resolve in dispatch order; every wait is bounded, and one that runs past `limit` polls sets *err
-// and gives up (the host reports the solve as failed), so every wave exits.
+// the diagonal). A level is one launch forward and two backward (the products with the rows below
+// first), or one more each way where it has many one-block fronts beside wider ones: a front's
+// workgroups each take 128 of its rows (forward) or columns (backward) through its blocks in order,
+// and the one that finishes the rows or columns of a block forms that block's solution. A block's
+// solution formed elsewhere is waited for value by value: the values to come are marked PENDING, a
+// signalling NaN that no arithmetic produces, before the launch; the forming workgroup writes each
+// with a device-coherent atomic store and a waiting thread polls its own values until they are not
+// PENDING (no fence: each value is its own signal). A workgroup waits only on workgroups of its own
+// front placed earlier in the launch, so the waits resolve in dispatch order; every wait is bounded,
+// and one that runs past `limit` polls sets *err and gives up (the host reports the solve as
+// failed), so every wave exits.
 //
 // The products run on the FP64 matrix cores (16x16x4): 16 rows of L by 16 right-hand sides, the
 // right-hand sides of an equation side by side in memory (entry k of side r at k nr + r), so that
 // every entry of L is read once for all of them. One right-hand side uses one column of sixteen:
-// 64 entries of L cost an MFMA either way, which is still above what memory delivers, and each
-// side's sums run in the same order however many are solved together: the same bits.
+// 64 entries of L cost an MFMA either way, some 2.4e12 entries a second, above the 1.2e12 (FP32) that
+// memory delivers, and each side's sums run in the same order however many are solved together: the
+// same bits.
 //
 // Bound: the top levels' chains of blocks, each a wait, two 128 x 128 products and a publication: 5 us
 // a block backward, 6 us forward (FP64, the 36^3 cube's root of 49 blocks), and below them the
 // levels' launches. Measured against a launch a block on the vector units, with a launch of one workgroup
 // a front to gather and one to start each level: 8 right-hand sides of the 20 x 23 x 17 hex8 block
-// 2.78 -> 0.76 ms; a refined solve of 16 vectors on the mixed factor of the 13^3 tet10 block 25.0 ->
-// 5.6 ms; one right-hand side of the 36^3 cube (one launch a level before, too) 3.60 -> 2.22 ms.
+// 2.78 -> 0.61 ms; a refined solve of 16 vectors on the mixed factor of the 13^3 tet10 block 25.0 ->
+// 5.1 ms; one right-hand side of the 36^3 cube (one launch a level before, too) 3.60 -> 2.12 ms. One-block
+// fronts with up to 512 rows below took their products in k_bwd itself at first, a launch less for
+// many levels: 0.70, 5.5 and 2.23 ms (one workgroup a front is too few waves for its rows).
 #pragma once
 
 #include <type_traits>
@@ -45,7 +49,6 @@ constexpr int SNB = 128;       // columns of a solve block (the factorization's 
 constexpr int SRHS = 16;       // right-hand sides of one product
 constexpr int MAX_RHS = 64;    // right-hand sides one solve pass handles (the host splits larger blocks)
 constexpr int STHREADS = 512;  // threads of a solve workgroup: eight waves of 16 rows or columns
-constexpr int BELOW_FUSE = 512;  // rows below a one-block front up to which k_bwd takes its products itself
 // A block solution not yet formed: a signalling NaN, which no arithmetic result is.
 constexpr uint64_t PENDING = 0x7FF0DEAD0000BEEFull;
 
@@ -426,16 +429,14 @@ __global__ __launch_bounds__(STHREADS) void k_bwd_below(const Item* __restrict__
   }
 }
 
-// Backward, item (f, a = jb, b = fused): the columns of block jb lose L(b, jb)^T x_b for every later
-// block b, last first, then x_jb = Inv_jb^T z_jb. Fused (a front of one block with few rows below):
-// the products with the rows below are taken here, each wave a 16-column block over its share of the
-// rows. A front's items are in decreasing jb, so the workgroup forming a block's x precedes every
-// one waiting for it.
+// Backward, item (f, a = jb): the columns of block jb lose L(b, jb)^T x_b for every later block b, last
+// first, then x_jb = Inv_jb^T z_jb. A front's items are in decreasing jb, so the workgroup forming a block's
+// x precedes every one waiting for it.
 template <typename T, int NG>
 __global__ __launch_bounds__(STHREADS) void k_bwd(const Item* __restrict__ items, const FrontDev* __restrict__ fronts,
                                                   const T* __restrict__ L, const T* __restrict__ Inv,
-                                                  const int32_t* __restrict__ rows, const double* __restrict__ z,
-                                                  double* xp, int nr, int nitems, int32_t* err, int64_t limit) {
+                                                  const double* __restrict__ z, double* xp, int nr, int nitems,
+                                                  int32_t* err, int64_t limit) {
   constexpr int KI = SNB / 16;  // steps of 16 rows
   __shared__ double Xs[SNB][SRHS * NG];
   const int grp = blockIdx.x / nitems;
@@ -460,26 +461,6 @@ __global__ __launch_bounds__(STHREADS) void k_bwd(const Item* __restrict__ items
       const int j = 16 * wave + q + 4 * v;
       zv[g][v] = (j < pw && 16 * g + r < sd.n) ? z[(int64_t)(F.col0 + j0 + j) * nr + sd.n0 + 16 * g + r] : 0.0;
     }
-  if (it.b) {
-    // column blocks up to the next power of two, the waves left over sharing the rows
-    const int nc = (pw + 15) / 16, cp = nc <= 1 ? 1 : (nc <= 2 ? 2 : (nc <= 4 ? 4 : 8)), rg = 8 / cp;
-    v4d acc[1][NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) acc[0][g] = v4d{0, 0, 0, 0};
-    const int cb = wave & (cp - 1);
-    if (cb < nc) below_products<T, NG, 1, 4>(acc, F, L, rows, xp, sd, 16 * cb, wave / cp, rg, lane);
-    to_lds<NG>(Xs, acc[0], 16 * wave, SNB, lane);
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (wave < nc) {
-          double s = Xs[16 * wave + q + 4 * v][16 * g + r];
-          for (int k = 1; k < rg; ++k) s += Xs[16 * (wave + cp * k) + q + 4 * v][16 * g + r];
-          zv[g][v] -= s;
-        }
-  }
   // four rows of KI steps of a column: block b of L, or the block's inverse
   auto fetch = [&](int b, double (&a)[KI][4]) {
     const int c0 = b * SNB, pb = min(SNB, F.w - c0);
@@ -635,14 +616,13 @@ __global__ __launch_bounds__(ONE_THREADS) void k_fwd_one(const Item* __restrict_
   }
 }
 
-// Backward, item (f, b = fused): x = Inv^T (y - L21^T x_below), the products with the rows below taken
-// here (fused) or before (k_bwd_below): each wave a 16-column block over its share of the rows, the waves
-// left over by a narrow front sharing them.
+// Backward, item (f): x = Inv^T z.
 template <typename T, int NG>
-__global__ __launch_bounds__(STHREADS, NG == 1 ? 4 : 2) void k_bwd_one(
-    const Item* __restrict__ items, const FrontDev* __restrict__ fronts, const T* __restrict__ L,
-    const T* __restrict__ Inv, const int32_t* __restrict__ rows, const double* __restrict__ z, double* xp, int nr,
-    int nitems) {
+__global__ __launch_bounds__(STHREADS, NG == 1 ? 4 : 2) void k_bwd_one(const Item* __restrict__ items,
+                                                                       const FrontDev* __restrict__ fronts,
+                                                                       const T* __restrict__ Inv,
+                                                                       const double* __restrict__ z, double* xp, int nr,
+                                                                       int nitems) {
   constexpr int KI = SNB / 16;
   __shared__ double Xs[SNB][SRHS * NG];
   const int grp = blockIdx.x / nitems;
@@ -651,7 +631,6 @@ __global__ __launch_bounds__(STHREADS, NG == 1 ? 4 : 2) void k_bwd_one(
   const FrontDev F = fronts[it.f];
   const int w = F.w, nc = (w + 15) / 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const int cp = nc <= 1 ? 1 : (nc <= 2 ? 2 : (nc <= 4 ? 4 : 8)), rg = 8 / cp;
   const int h = 16 * wave;
   v4d zv[NG];
 #pragma unroll
@@ -661,14 +640,6 @@ __global__ __launch_bounds__(STHREADS, NG == 1 ? 4 : 2) void k_bwd_one(
       const int j = h + q + 4 * v;
       zv[g][v] = (j < w && 16 * g + r < sd.n) ? z[(int64_t)(F.col0 + j) * nr + sd.n0 + 16 * g + r] : 0.0;
     }
-  if (it.b) {  // uniform
-    v4d acc[1][NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) acc[0][g] = v4d{0, 0, 0, 0};
-    const int cb = wave & (cp - 1);
-    if (cb < nc) below_products<T, NG, 1, 2>(acc, F, L, rows, xp, sd, 16 * cb, wave / cp, rg, lane);
-    to_lds<NG>(Xs, acc[0], h, SNB, lane);
-  }
   // the inverse's columns (zero above its diagonal: rows h on), in flight over the barrier
   T inv[KI][4];
   {
@@ -680,19 +651,6 @@ __global__ __launch_bounds__(STHREADS, NG == 1 ? 4 : 2) void k_bwd_one(
       for (int s = 0; s < 4; ++s)
         inv[k][s] = buf_load<T>(rs, (16 * k >= h && 16 * k + 4 * q + s < w) ? lo + s * (uint32_t)sizeof(T) : 0x80000000u,
                                 16 * k * (uint32_t)sizeof(T));
-  }
-  __syncthreads();
-  if (it.b) {
-    if (wave < nc)
-#pragma unroll
-      for (int g = 0; g < NG; ++g)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          double s = Xs[h + q + 4 * v][16 * g + r];
-          for (int k = 1; k < rg; ++k) s += Xs[h + 16 * cp * k + q + 4 * v][16 * g + r];
-          zv[g][v] -= s;
-        }
-    __syncthreads();  // every partial sum read
   }
   if (wave < nc) to_lds<NG>(Xs, zv, h, w, lane);
   __syncthreads();

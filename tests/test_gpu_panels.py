@@ -55,8 +55,7 @@ SHAPES = [(1, 2, 1), (15, 17, 16), (16, 31, 33), (63, 65, 15), (64, 66, 64), (12
           (200, 96, 129), (257, 191, 65), (300, 130, 200)]
 
 
-# the last: fronts of 33 and 40 columns with some 600 rows below, more than the backward pass takes in one
-# launch with the block itself
+# the last: fronts of 33 and 40 columns with 130 to 600 rows below
 TREES = [(15, 17, 80, 130), (16, 31, 65, 120), (63, 65, 64, 129), (64, 66, 100, 130),
          (127, 129, 97, 150), (128, 130, 129, 128), (200, 96, 129, 257), (257, 191, 129, 150), (40, 33, 200, 900)]
 
