@@ -180,7 +180,9 @@ struct Program {
 };
 
 // Waves of a TRSM launch from which its workgroups take TRSM_WAVES each: four a SIMD (1 024 SIMDs)
-// keep the chip as busy either way, and a quarter of the items is read.
+// keep the chip as busy either way, and a quarter of the items is read. Measured: single waves
+// throughout, the 80^3 cube's mixed factor's rows below 20.5 -> 25.2 ms; four a workgroup
+// throughout, the cantilever's FP64 step 1.3 % longer; lines at 1 024 and 2 048 within 0.6 % of this one.
 constexpr i64 TRSM_WIDE = 4096;
 
 // Side-stream panel updates (Launch.pad of their UPDATE and REDUCE launches): one variant for the
@@ -200,14 +202,19 @@ static_assert(fc::SNB == fc::NB, "solve blocks are the factorization's panels");
 
 // In a level with wider fronts, one-block fronts of up to this many workgroups in all take the wide
 // fronts' launch (each launch of a level is another dependent step); more take one of their own,
-// whose kernel keeps more workgroups on a CU.
-constexpr i64 ONE_FEW = 256;
+// whose kernel keeps more workgroups on a CU. Measured: against a line at 256, 16 refined vectors of the
+// 13^3 tet10 block 2.9 % shorter and a batch of 8 models 2.3 %; at 64 or 0, 8 sides of the 20 x 23 x 17
+// block 6 % longer; at 4 096 one side of the 36^3 cube 2 % longer, without a line that of the 80^3 one 10 %.
+constexpr i64 ONE_FEW = 1024;
 // One-block fronts' forward workgroups take ONE_ROWS rows, or a quarter of that in launches of fewer
 // than ONE_MANY workgroups (a workgroup takes its rows 64 at a time, several memory round trips
-// each; every one forms the block's y again).
+// each; every one forms the block's y again). Measured: ONE_ROWS throughout, 8 sides of the
+// 20 x 23 x 17 block 7.6 % longer; a quarter throughout, one side of the 80^3 cube's mixed factor 3.0 %.
 constexpr i64 ONE_MANY = 2048;
 // Launches of the products with the rows below take 16 columns a workgroup instead of 32 where there are
-// fewer than this many.
+// fewer than this many. Measured: 32 throughout, 8 sides of the 20 x 23 x 17 block 2.0 % and 16 vectors of
+// the 13^3 tet10 block 2.5 % longer; 16 throughout, one side of the 80^3 cube's mixed factor 3.2 %; lines at 256
+// and 1 024 within the noise of this one.
 constexpr i64 SOLVE_FEW = 512;
 
 // lower pairs (i >= j) of rows [r0, r1) x columns [c0, c1)
@@ -229,11 +236,15 @@ constexpr i64 SPLIT_MIN_K = 512;
 // GEMM launches of at most this many 128 x 128 tiles take 64 x 64 ones instead (four times the
 // workgroups, a quarter of the work each): below one tile a CU a launch's time is its tile's own
 // chain of stages, and one FP64 tile 128 deep is 14 us of a CU's matrix cores. Measured, launches of
-// the 40 x 8 x 8 cantilever's FP64 factor 46 -> 17 us; BF16 ones of the 40^3 cube at most 18 us.
+// the 40 x 8 x 8 cantilever's FP64 factor 46 -> 17 us; BF16 ones of the 40^3 cube at most 18 us. The
+// line: none, the cantilever and the 28^3 cube in FP64 21 to 22 % longer, the 40^3 mixed one 3.7 %; at
+// 384, those within 0.9 %, the 80^3 mixed factor 1.9 % longer.
 constexpr i64 GB_FEW = 192;
 
-// Workgroups an extend-add launch is divided into where its columns allow (four a CU).
-constexpr i64 EA_ITEMS = 1024;
+// Workgroups an extend-add launch is divided into where its columns allow (sixteen a CU, twice what one
+// holds at a time: their weights differ). Measured, FP64 cantilever, 28^3 cube and the batch of 8 models: at 1 024
+// 2.2, 1.9 and 1.8 % longer, at 256 another 2, 0.3 and 0.7; at 16 384 as here; the 80^3 factor does not care.
+constexpr i64 EA_ITEMS = 4096;
 
 // One GEMM launch of `tiles` (kind: UPDATE or SYRK), split along k when the tiles are
 // too few, followed by the launch that reduces the pieces.
