@@ -853,13 +853,12 @@ __device__ __forceinline__ zd ldl_chain(zd sum, const zd* b, int cnt) {
   return sum;
 }
 
-constexpr int LDL_BW_CAP = 3840;    // products of one column held in LDS (two such buffers)
-constexpr int LDL_BW_SMALL = 1024;  // the same for levels whose supernodes have no more rows
+constexpr int LDL_BW_CAP = 3840;  // products of one column held in LDS (two such buffers)
 
 // The backward pass (cholesky.rs:982-1030) for the supernodes of one level (sn[blockIdx.x]),
 // levels from the root down: a supernode's unknowns are its own and its sums read only its
 // ancestors' (final) unknowns, so the supernodes of a level are independent. Each sum runs in
-// the reference's order on one lane. With m <= cap (<= CAP), waves 1.. stage the next column's
+// the reference's order on one lane. With m <= cap (<= LDL_BW_CAP), waves 1.. stage the next column's
 // products while lane 0 runs the current column's sum: the one product that needs the unknown
 // being finished (its row is the current column's q) is left to lane 0, which forms it first.
 // Larger supernodes stage each column in chunks before its sum.
@@ -869,18 +868,21 @@ constexpr int LDL_BW_SMALL = 1024;  // the same for levels whose supernodes have
 // (the unknowns of all m rows, the pivot kinds) is taken to LDS once, and PRE entries a thread of the
 // column after the staged one are in flight, so that short columns are not bound by two or three
 // loads one behind another instead (2 % of the pass there).
-// CAP = LDL_BW_SMALL leaves room for several workgroups a CU where a level has many small supernodes.
-template <typename T, int CAP>
+// One workgroup a CU: a form of 1 024 rows for levels of small supernodes, with room for several, took as
+// long (tet10 blocks of 8 to 12 cells a side, hex8 of 16 and 20, real and complex: within 2 % either way),
+// the few supernodes at the top being the pass.
+template <typename T>
 __global__ __launch_bounds__(256) void k_ldlt_solve_bwd(const int64_t* __restrict__ sn, const LdlSupernode* __restrict__ S,
                                                        const int64_t* __restrict__ rows_all, const T* __restrict__ val,
                                                        const int8_t* __restrict__ piv, const int32_t* __restrict__ order,
                                                        T* __restrict__ x, T* __restrict__ ywork, int cap) {
 #pragma clang fp contract(off)
+  constexpr int CAP = LDL_BW_CAP;
   constexpr int PL = CAP + 32;                                          // one buffer of products
   constexpr int ROOM = (160 * 1024 - 256 - CAP) / (int)sizeof(T) - 2 * PL;  // entries of LDS left for the unknowns
   constexpr int VC = ROOM < CAP ? ROOM : CAP;
   constexpr int ST = 192;       // staging threads
-  constexpr int PRE = 6;        // entries a thread holds of a column (6 x 192 > LDL_BW_SMALL)
+  constexpr int PRE = 6;        // entries a thread holds of a column
   const LdlSupernode K = S[sn[blockIdx.x]];
   const int m = K.m, w = K.w;
   const T* t = val + K.voff;

@@ -960,7 +960,6 @@ struct fc_ldlt {
   int32_t* order = nullptr;
   int64_t* sn = nullptr;           // supernodes by level
   std::vector<int64_t> lvl_ptr;
-  std::vector<int64_t> lvl_rows;   // most rows of a supernode of each level
   bool complex = false;            // values are (re, im) pairs: complex-symmetric LDL^T
   int64_t* perm = nullptr;         // postorder position -> original equation (device)
   fc::LdlUpdate* U = nullptr;      // updates and their relative maps, for the forward gather
@@ -2283,10 +2282,6 @@ int ldlt_numeric(const fc_symbolic* h, const T* upper_val, uint64_t nnz, int32_t
     int64_t* dsn = dupload(P.lvl_sn, stq);
     F->sn = dsn;
     F->lvl_ptr = P.lvl_ptr;
-    F->lvl_rows.assign(P.lvl_ptr.size() - 1, 0);
-    for (size_t l = 0; l + 1 < P.lvl_ptr.size(); ++l)
-      for (i64 q = P.lvl_ptr[l]; q < P.lvl_ptr[l + 1]; ++q)
-        F->lvl_rows[l] = std::max<i64>(F->lvl_rows[l], P.sn[P.lvl_sn[q]].m);
     double* dscale = dupload(scale, stq);
     T* daval = dalloc<T>((size_t)std::max<uint64_t>(nnz, 1));
     T* dwork = dalloc<T>((size_t)std::max<i64>(P.work, 1));
@@ -2448,9 +2443,8 @@ void ldlt_passes(const fc_ldlt* f, const T* fv, T* dx, T* dz, T* dyw, hipStream_
   for (i64 l = (i64)f->lvl_ptr.size() - 2; l >= 0; --l) {
     const i64 cnt = f->lvl_ptr[l + 1] - f->lvl_ptr[l];
     if (cnt > 0)
-      (f->lvl_rows[l] <= fc::LDL_BW_SMALL ? fc::k_ldlt_solve_bwd<T, fc::LDL_BW_SMALL>
-                                          : fc::k_ldlt_solve_bwd<T, fc::LDL_BW_CAP>)<<<(unsigned)cnt, 256, 0, st>>>(
-          f->sn + f->lvl_ptr[l], f->S, f->rows, fv, f->piv, f->order, dx, dyw, cap);
+      fc::k_ldlt_solve_bwd<T><<<(unsigned)cnt, 256, 0, st>>>(f->sn + f->lvl_ptr[l], f->S, f->rows, fv, f->piv, f->order, dx,
+                                                            dyw, cap);
   }
 }
 

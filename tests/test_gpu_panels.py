@@ -13,7 +13,7 @@ The matrices are 3 I plus a symmetric random part of norm below 1.2 (condition b
 backward-stable factor or solve of n <= 1 206 columns is off by at most about n u times that: 4e-13 in
 FP64 (1e-12 asserted, the comparison being as inexact) and, the larger ones' condition being below 2.2,
 1.7e-4 in FP32. Every side of a block solve is the bits of the same side alone. The LDL^T solve's columns at its own limits (a panel of 64
-columns, 1 024 rows in the small form of the backward pass) are the oracle's bits."""
+columns, the 1 152 entries of a column held ahead in the backward pass) are the oracle's bits."""
 import numpy as np
 import pytest
 
@@ -114,7 +114,8 @@ def test_block_solves_are_the_bits_of_lone_ones(gpu, shape, precision, nrhs):
         assert np.array_equal(x, f.solve(b))
 
 
-@pytest.mark.parametrize("shape", [(1, 2, 1), (63, 65, 64), (64, 129, 66), (3, 200, 130), (2, 40, 990), (2, 40, 1030)],
+@pytest.mark.parametrize("shape", [(1, 2, 1), (63, 65, 64), (64, 129, 66), (3, 200, 130), (2, 40, 990), (2, 40, 1030),
+                                   (2, 40, 1160)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_ldlt_columns_are_the_oracles_bits(gpu, shape):
     a = cliques(*shape, shift=0.1)  # indefinite: 2 x 2 pivots

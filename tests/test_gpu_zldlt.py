@@ -94,9 +94,9 @@ def test_singular_complex_matrix_and_argument_errors(gpu):
 @pytest.mark.parametrize("values", ["real", "dominant"])
 def test_tall_complex_supernodes_match_the_oracle_bit_for_bit(gpu, monkeypatch, wa, rows, wd, chunk, values):
     """A block of wa columns with `rows` rows below it in a dense block of wd columns: supernodes of more
-    rows than the backward pass's small form takes (1 024), than the unknowns its LDS has room for beside
-    two columns of products (2 240 complex ones) and, with FC_LDLT_SOLVE_ROWS, than it stages of a
-    column at a time. A 2 x 2 pivot is chosen between two computed values of one entry, a tie to a
+    rows than the backward pass holds ahead of a column (1 152), than the unknowns its LDS has room for
+    beside two columns of products (2 240 complex ones) and, with FC_LDLT_SOLVE_ROWS, than it stages
+    of a column at a time. A 2 x 2 pivot is chosen between two computed values of one entry, a tie to a
     rounding in which the last bit of hypot decides, and libraries differ in it. The values are therefore
     real, where the modulus is exact and a third of the pivots are 2 x 2, or complex with a diagonal that
     every search stops at; the right-hand sides are complex."""
