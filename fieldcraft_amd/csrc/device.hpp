@@ -23,8 +23,10 @@ static_assert(sizeof(FrontDev) == 56, "FrontDev layout");
 
 // Strided runs of loads (and stores) through a buffer resource: the lane's part of the address
 // is one VGPR offset and each access's part a scalar, so a run of independent accesses needs no
-// 64-bit address per access. Raw resource (byte offsets, stride 0); every access made through
-// it is in bounds by construction, the record count only has to cover the lane offsets.
+// 64-bit address per access. Raw resource (byte offsets, stride 0) of 2^31 - 1 bytes: an access that
+// is not to happen takes the lane offset 2^31, which the buffer unit's range check turns into a read of 0
+// or no store, and with it no branch. Every other lane offset has to lie in the array by the kernel's own
+// indexes: the resource ends where its 2^31 - 1 bytes do, not where the array does.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
 }

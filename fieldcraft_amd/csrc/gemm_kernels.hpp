@@ -1,17 +1,17 @@
 // Dense kernels of a front's partial factorization on the matrix cores (gfx950).
 //
-// Every GEMM-shaped step of the numeric phase is one item of one kernel, k_gemm:
+// The Schur products of the numeric phase are items of one kernel, k_gemm (k_gemm_b16 in the mixed form):
 //   panel update   L[r.., c0..c1) -= L[r.., 0..c0) L[c0..c1, 0..c0)^T      (G_SUB)
 //   update matrix  U[i.., j..)     = -L[W+i.., 0..W) L[W+j.., 0..W)^T        (G_NEG)
-// (the rows below a panel's diagonal block are panel_kernels.hpp's). A launch with few output tiles is split along k: each piece writes its partial tile (G_PART) and
-// k_reduce_parts adds the pieces in a fixed order, so results do not depend on scheduling.
+// (a panel's diagonal block and the rows below it are panel_kernels.hpp's). A launch with few
+// output tiles is split along k: each piece writes its partial tile (G_PART) and k_reduce_parts adds
+// the pieces in a fixed order, so results do not depend on scheduling.
 //
 // Tile: TB x TB per workgroup of 4 waves (128, or 64 in launches of few tiles: GB_FEW), each wave a
 // quarter as blocks of the 16x16x4 MFMA; k staged in LDS (16 at a time, 32 for the smaller tile),
-// the next stage prefetched into registers while
-// the current one is multiplied (one barrier a stage). The MFMA's first operand is taken from
-// the j side so that a lane's output column index runs along C's rows: 16 lanes store 16
-// consecutive rows of a column (coalesced, C is column-major).
+// the next stage prefetched into registers while the current one is multiplied (one barrier a
+// stage). The MFMA's first operand is taken from the j side so that a lane's output column index
+// runs along C's rows: 16 lanes store 16 consecutive rows of a column (coalesced, C is column-major).
 #pragma once
 
 #include "device.hpp"

@@ -300,9 +300,9 @@ void add_gemm(Program& p, const std::vector<Tile>& tiles, int kind, i64 level, i
   p.part_size = std::max(p.part_size, part);
 }
 
-// Fronts whose dense steps one workgroup of k_small_fronts takes: at most SMALL_W columns (one
-// wave's diagonal block), and an update matrix of at most SMALL_SYRK multiply-adds (the part
-// that sets a front's time there: a front above it is faster on the tiled launches).
+// Fronts whose dense steps one workgroup of k_small_fronts takes: at most SMALL_W columns (a
+// diagonal block of one step a wave), and an update matrix of at most SMALL_SYRK multiply-adds (the
+// part that sets a front's time there: a front above it is faster on the tiled launches).
 bool is_small(const fc::Symbolic& s, i64 f) {
   const double w = (double)s.f_w[f], mu = (double)(s.f_m[f] - s.f_w[f]);
   return s.f_w[f] <= fc::SMALL_W && s.f_m[f] - s.f_w[f] <= fc::SMALL_MU && 0.5 * mu * mu * w <= fc::SMALL_SYRK;

@@ -336,7 +336,7 @@ Failure analyze(i64 n, const i64* ptr, const i64* idx, i64 max_entries, const Pl
   // height spread them with the irregularity of what hangs below. It also ends an update matrix's
   // life one level after its front's. Against levels by height: the 28^3 cube's factor and solve
   // 248 -> 235 launches, 10.56 -> 10.11 ms, 0.79 -> 0.64 GB of update matrices; the 40 x 8 x 8
-  // cantilever's 80 -> 64 launches, 2.31 -> 1.85 ms; 64 small models together 152 -> 101, 8.78 -> 7.18 ms.
+  // cantilever's 80 -> 64 launches, 2.31 -> 1.85 ms; 8 small models with 64 load cases 152 -> 101, 8.78 -> 7.18 ms.
   s.f_level.assign(nf, 0);
   for (i64 f = nf; f-- > 0;)
     if (s.f_parent[f] != NONE) s.f_level[f] = s.f_level[s.f_parent[f]] + 1;
@@ -384,8 +384,7 @@ Failure analyze(i64 n, const i64* ptr, const i64* idx, i64 max_entries, const Pl
   }
   // The solves' per-front vectors (M - W entries a right-hand side) in an arena of their own,
   // with the same level lifetimes: a front's contribution is written at its level and read by
-  // its parent (forward); on the way back a level's blocks are written and read within the level.
-  // 8-entry blocks keep every front's vector aligned to 64 bytes.
+  // its parent, on the way up only. 8-entry blocks keep every front's vector aligned to 64 bytes.
   s.f_soff.assign(nf, 0);
   {
     Arena arena;

@@ -1,9 +1,9 @@
 """GPU parity of the small-front launch (a front of at most 64 columns taken whole by one
 workgroup) against the oracle, through the C ABI: a dense 64-column front alone (FP64 values and
-solutions within 1e-12); fronts whose FP32 attempt meets a small pivot (below 1e-3 |A_jj|) and are
-factored again in FP64 (every value of the FP32-storage forms within FP32 rounding of the oracle's
-factor of the FP32-rounded matrix, where FP32 arithmetic would be off by 1e-3); a failing pivot inside a small front, named by its
-column in every precision."""
+solutions within 1e-12); fronts with a small pivot (below 1e-3 |A_jj|), every value of the FP32-storage
+forms within FP32 rounding of the oracle's factor of the FP32-rounded matrix (the blocks are factored in
+FP64 arithmetic; FP32 would be off by 1e-3); a failing pivot inside a small front, named by its column
+in every precision."""
 import numpy as np
 import pytest
 
@@ -92,12 +92,11 @@ def test_a_failing_pivot_in_a_small_front_is_named(gpu, precision):
 @pytest.mark.parametrize("precision", ["fp32", "mixed"])
 def test_fp32_diagonal_blocks_of_every_quarter_shape(gpu, n, precision):
     """A dense front of n columns (wider than a small front) factored by the tiled kernels: its
-    128-column panels' FP32 diagonal blocks go in 32-column quarters, and these widths give a
-    last panel of 1, 32, 33, 40, 72, 122 columns and halves of every shape (a lone quarter, a
-    quarter and a part, two whole ones). Every value within 2e-6 of the oracle's factor of the
-    FP32-rounded matrix (normwise; 1e-4 for the mixed form, whose panel updates are BF16 split
-    products), and its inverse blocks right: the refined solve reaches berr <= 1e-12. A wrong
-    quarter product would be off by O(1)."""
+    128-column panels' diagonal blocks go by steps of 16 columns, and these widths give a last panel of
+    1, 32, 33, 40, 72, 122 columns: whole steps and parts of one. Every value within 2e-6 of the oracle's
+    factor of the FP32-rounded matrix (normwise; 1e-4 for the mixed form, whose panel updates are BF16
+    split products), and its inverse blocks right: the refined solve reaches berr <= 1e-12. A wrong
+    step would be off by O(1)."""
     a = random_spd(n, 1.0, 100 + n)
     sym, _, f, (nn, ptr, idx, val) = factor_both(a, precision)
     assert sym.info()["kind_flops"]["small"] == 0
