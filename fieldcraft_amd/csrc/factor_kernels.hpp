@@ -78,8 +78,8 @@ __global__ void k_fill(T* __restrict__ p, int64_t len, T v) {
 // rows of each in flight. Bound: HBM, 12 bytes a child's FP32 entry (20 FP64) and the row maps; in
 // levels of few columns, the chain of a workgroup's ranges (three memory round trips each). Taken
 // as one flat range of 8 columns by the whole workgroup, with a barrier after each child and
-// selects to find an entry's column, a launch of the cantilever's FP64 factor took 64 us (now 9), of
-// the 28^3 cube's 91 us (57), of the 40^3 cube's mixed one 136 us (100).
+// selects to find an entry's column, a launch of the cantilever's FP64 factor took 64 us (now 7), of
+// the 28^3 cube's 91 us (48), of the 40^3 cube's mixed one 136 us (97).
 template <typename T>
 __global__ __launch_bounds__(256) void k_extend_add(const Item* __restrict__ items, const EaRange* __restrict__ ranges,
                                                     const FrontDev* __restrict__ fronts,

@@ -1,8 +1,9 @@
 // Tall-skinny kernels of the shift-invert block Lanczos on the device (gfx950, wave64): the
 // basis Q and its M products MQ are n x m column-major in HBM; a block W is n x b (b <= 8).
 // Both kernels stream the basis once per call: HBM-bound on large problems, a few microseconds of
-// launch and reduction on small ones. Six modes of a tet10 block of 5 x 7 x 9 cells (some 9 000 unknowns) took 26.6 ms with
-// one copy and one synchronization for each set of coefficients and chunks of 4 096 rows, now 15.2.
+// launch and reduction on small ones. Six modes of a tet10 block of 5 x 7 x 9 cells (some 9 000
+// unknowns) took 26.6 ms with one copy and one synchronization for each set of coefficients and
+// chunks of 4 096 rows, now 14.1.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -55,7 +55,7 @@ __device__ __forceinline__ void root_pair(double p, double& d, double& rd) {
 // trailing update S(r, j) -= P(r) L(j)^T (rows below, and identity rows already started) goes
 // through the 16x16x4 MFMA, row block r by wave r. Measured, a 128-column block: 90 us with a wave's
 // 8 x 8 lane grid passing columns through LDS shuffles on 32-column quarters, and products between
-// the quarters (FP32 arithmetic: 60 us); 38 us in this form, the pivots' chain 12 us of it, the tiles 9.
+// the quarters (FP32 arithmetic: 60 us); 37 us in this form, the pivots' chain some 12 us of it, the tiles 9.
 template <int NMAX>
 using DiagX = double[NMAX / DB][DB][DB + 1];
 

@@ -236,14 +236,15 @@ constexpr i64 SPLIT_MIN_K = 512;
 // GEMM launches of at most this many 128 x 128 tiles take 64 x 64 ones instead (four times the
 // workgroups, a quarter of the work each): below one tile a CU a launch's time is its tile's own
 // chain of stages, and one FP64 tile 128 deep is 14 us of a CU's matrix cores. Measured, launches of
-// the 40 x 8 x 8 cantilever's FP64 factor 46 -> 17 us; BF16 ones of the 40^3 cube at most 18 us. The
-// line: none, the cantilever and the 28^3 cube in FP64 21 to 22 % longer, the 40^3 mixed one 3.7 %; at
-// 384, those within 0.9 %, the 80^3 mixed factor 1.9 % longer.
+// the 40 x 8 x 8 cantilever's FP64 factor 46 -> 19 us. The line: without one, the cantilever and the
+// 28^3 cube in FP64 take 21 to 22 % longer, the 40^3 mixed one 3.7 %; at 384, those within 0.9 %, the
+// 80^3 mixed factor 1.9 % longer.
 constexpr i64 GB_FEW = 192;
 
-// Workgroups an extend-add launch is divided into where its columns allow (sixteen a CU, twice what one
-// holds at a time: their weights differ). Measured, FP64 cantilever, 28^3 cube and the batch of 8 models: at 1 024
-// 2.2, 1.9 and 1.8 % longer, at 256 another 2, 0.3 and 0.7; at 16 384 as here; the 80^3 factor does not care.
+// Workgroups an extend-add launch is divided into where its columns allow (sixteen a CU, twice what
+// one holds at a time: their weights differ). Measured, FP64 cantilever, 28^3 cube and the batch of
+// 8 models: at 1 024 2.2, 1.9 and 1.8 % longer, at 256 another 2, 0.3 and 0.7; at 16 384 as here; the
+// 80^3 factor takes the same time with any of them.
 constexpr i64 EA_ITEMS = 4096;
 
 // One GEMM launch of `tiles` (kind: UPDATE or SYRK), split along k when the tiles are

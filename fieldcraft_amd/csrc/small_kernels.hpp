@@ -15,9 +15,10 @@
 // BF16 copies for them, since no product of the tiled path reads a small front.
 //
 // Bound: a workgroup's own chain (diagonal block, rows, products), since a level has few fronts of
-// equal weight. Rows as one thread each and products on the vector units took 266 us a launch on
-// the 40 x 8 x 8 cantilever's FP64 factor and 192 us on the 40^3 cube's mixed one (the FP64 row
-// code spilled); on the matrix cores 69 and 89 us.
+// equal weight. Rows as one thread each and products on the vector units took 266 us in the
+// largest launch of the 40 x 8 x 8 cantilever's FP64 factor and 192 us of the 40^3 cube's mixed one (the
+// FP64 row code spilled); on the matrix cores 74 and 104 us, with the levels counted from the root and
+// so more fronts in them (41 and 66 on average).
 #pragma once
 
 #include "panel_kernels.hpp"
