@@ -244,7 +244,7 @@ def main():
         log("bench: fp64 leg")
         tune("fp64")
         legs["fp64"] = run_leg(CH, sym, dvals.data_ptr(), A, b.data_ptr(), x.data_ptr(), p.n, "fp64", args.steps,
-                               args.warmup, [], breakdown=breakdown)
+                               args.warmup, profile if args.form == "fp64" else [], breakdown=breakdown)
         x64 = x.cpu().numpy().copy()
         log(f"bench: fp64 {legs['fp64']}")
     form = args.form
